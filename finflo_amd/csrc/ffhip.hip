@@ -1423,16 +1423,15 @@ __global__ void __launch_bounds__(128) k_residual(Prm p, Blk b, WallDev wd)
 }
 
 // Residual with every face flux formed once.  A workgroup is a tile of RI x RJ cells in
-// (I,J) that marches over RK consecutive K-planes.  At each plane a lane forms the K-face
-// above its cell (kept in registers: it is the lower K-face of the next plane), its lower
-// I-face and its lower J-face; the tile's upper I- and J-faces are formed by two waves in an
+// (I,J) that marches over RKC consecutive K-planes (RKW in the k-omega form).  At each plane
+// a lane forms its cell's lower I-face and lower J-face, then the K-face above it (kept in
+// LDS: it is the lower K-face of the next plane); the tile's upper I- and J-faces are formed by two waves in an
 // extra phase.  I- and J-faces meet their two cells through LDS.  A face flux is the same
 // function of the same operands whichever cell forms it, so the differences are those of
 // k_residual bit for bit.
-constexpr int RI = 64, RJ = 4, RKC = 8;
-static_assert(RJ >= 2 && RJ <= RI, "the tile's upper I-faces are formed by the lanes of row 1");
+constexpr int RI = 32, RJ = 8;     // the built-in (I, J) tile (launch_residual)
 
-template <int IFLUX, bool FNS = false, int RI = ::RI, int RJ = ::RJ, int RKC = ::RKC>
+template <int IFLUX, bool FNS, int RI, int RJ, int RKC>
 __global__ void __launch_bounds__(RI * RJ) k_residual_tile(Prm p, Blk b, WallDev wd, TileGrid tg)
 {
     static_assert(RJ >= 2 && RI >= RJ, "the tile's upper faces need two rows and RI >= RJ");
@@ -4586,6 +4585,26 @@ int ff_turb(ff_ctx *c, int level, int block)
 // the same operands); they differ in occupancy, halo re-reads and how many workgroups a
 // small (coarse-level) block offers the 256 CUs.
 
+// The built-in shape: 32x8 (I, J) tiles of one K-plane, or of two where one plane per
+// workgroup would make more than RES_WGS1 workgroups.  A face flux takes a lone wave about
+// 4 us (divisions and loads in one long chain), and a workgroup of n planes runs 4n + 1 of
+// them one after another: short tiles keep that chain short and the chip full, at the price
+// of one more K-face per tile.  Measured (k-omega residual, us): 64x4x8 tiles / 32x8x1 /
+// 32x8x2 on 48x24x24 165 / 31 / 47, on 101x53x47 194 / 91 / 88, on 128x64x64 197 / 129 /
+// 133, on 160x80x80 354 / 277 / 266, on 192x96x96 551 / 475 / 459; laminar 118 / 23 / 33,
+// 143 / 70 / 67, 143 / 96 / 99, 258 / 191 / 185, 397 / 340 / 329.  The line lies between
+// 128x64x64 (2048 one-plane workgroups) and 160x80x80 (4000).
+constexpr int RES_WGS1 = 3072;
+template <typename K>
+static int launch_residual(ff_ctx *c, const char *name, K k1, K k2, const Prm &kp, const Blk &b,
+                           const WallDev &wd)
+{
+    const int nx = (b.imax + RI - 1) / RI, ny = (b.jmax + RJ - 1) / RJ;
+    const bool two = (long long)nx * ny * b.kmax > RES_WGS1;
+    const TileGrid tg = tile_grid(nx, ny, two ? (b.kmax + 1) / 2 : b.kmax);
+    return launch(c, name, two ? k2 : k1, dim3(NXCD * tg.per), dim3(RI * RJ), kp, b, wd, tg);
+}
+
 // the k-omega (kind 1) or laminar Roe (kind 0) residual kernel of shape s over block b
 template <int S>
 static int launch_shape(ff_ctx *c, bool kw, const Prm &kp, const Blk &b, const WallDev &wd)
@@ -4768,40 +4787,31 @@ static int residual_impl(ff_ctx *c, BlockRec *r, int level, int m2, double *resi
         if ((rc = walls())) return rc;
         if (level == 1 && (rc = inlout_impl(c, r, level))) return rc;
         const int sh = fns ? -1 : tuned_shape(c, true, kp, b, wr.wd);
-        if (sh >= 0) {
-            rc = launch_shape_any(c, sh, true, kp, b, wr.wd);
-        } else if (level >= 2) {
-            // the coarse levels' blocks are small: 32x4 tiles of two planes keep every CU busy
-            const TileGrid tg = tile_grid((b.imax + 31) / 32, (b.jmax + 3) / 4, (b.kmax + 1) / 2);
-            rc = launch(c, "k_residual_kw", k_residual_kw<32, 4, 2>, dim3(NXCD * tg.per), dim3(128),
-                        kp, b, wr.wd, tg);
-        } else {
-            const TileGrid tg = tile_grid((b.imax + 63) / 64, (b.jmax + 3) / 4, (b.kmax + 7) / 8);
-            dim3 g(NXCD * tg.per);
-            rc = fns ? launch(c, "k_residual_kw_ns", k_residual_kw<64, 4, 8, true>, g, dim3(256), kp, b, wr.wd, tg)
-                     : launch(c, "k_residual_kw", k_residual_kw<64, 4, 8>, g, dim3(256), kp, b, wr.wd, tg);
-        }
+        rc = sh >= 0 ? launch_shape_any(c, sh, true, kp, b, wr.wd)
+             : fns   ? launch_residual(c, "k_residual_kw_ns", k_residual_kw<RI, RJ, 1, true>,
+                                       k_residual_kw<RI, RJ, 2, true>, kp, b, wr.wd)
+                     : launch_residual(c, "k_residual_kw", k_residual_kw<RI, RJ, 1>,
+                                       k_residual_kw<RI, RJ, 2>, kp, b, wr.wd);
     } else {
         if (fns && (rc = gradients())) return rc;
         if ((rc = walls())) return rc;
         if (level == 1 && (rc = inlout_impl(c, r, level))) return rc;
+        const Prm kp = make_prm(&c->prm, level);
         const int sh = (fns || vl || c->residual_mode != FF_RESIDUAL_TILES) ? -1
-                       : tuned_shape(c, false, make_prm(&c->prm, level), b, wr.wd);
+                       : tuned_shape(c, false, kp, b, wr.wd);
         if (sh >= 0) {
-            rc = launch_shape_any(c, sh, false, make_prm(&c->prm, level), b, wr.wd);
+            rc = launch_shape_any(c, sh, false, kp, b, wr.wd);
         } else if (c->residual_mode == FF_RESIDUAL_TILES) {
-            const TileGrid tg = tile_grid((b.imax + RI - 1) / RI, (b.jmax + RJ - 1) / RJ,
-                                          (b.kmax + RKC - 1) / RKC);
-            dim3 g(NXCD * tg.per);
-            auto kern = fns ? (vl ? k_residual_tile<0, true> : k_residual_tile<1, true>)
-                            : (vl ? k_residual_tile<0> : k_residual_tile<1>);
-            rc = launch(c, fns ? "k_residual_tile_ns" : "k_residual_tile", kern, g,
-                        dim3(RI * RJ), make_prm(&c->prm, level), b, wr.wd, tg);
+            auto k1 = fns ? (vl ? k_residual_tile<0, true, RI, RJ, 1> : k_residual_tile<1, true, RI, RJ, 1>)
+                          : (vl ? k_residual_tile<0, false, RI, RJ, 1> : k_residual_tile<1, false, RI, RJ, 1>);
+            auto k2 = fns ? (vl ? k_residual_tile<0, true, RI, RJ, 2> : k_residual_tile<1, true, RI, RJ, 2>)
+                          : (vl ? k_residual_tile<0, false, RI, RJ, 2> : k_residual_tile<1, false, RI, RJ, 2>);
+            rc = launch_residual(c, fns ? "k_residual_tile_ns" : "k_residual_tile", k1, k2, kp, b, wr.wd);
         } else {
             auto kern = fns ? (vl ? k_residual<0, true> : k_residual<1, true>)
                             : (vl ? k_residual<0> : k_residual<1>);
             rc = launch(c, fns ? "k_residual_ns" : "k_residual", kern, cells_grid(b, 128),
-                        dim3(128), make_prm(&c->prm, level), b, wr.wd);
+                        dim3(128), kp, b, wr.wd);
         }
     }
     if (rc) return rc;
