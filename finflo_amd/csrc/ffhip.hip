@@ -30,6 +30,7 @@
 #include <cstring>
 #include <map>
 #include <tuple>
+#include <type_traits>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -3005,7 +3006,7 @@ __global__ void __launch_bounds__(TW) k_corr_st(Prm p, Blk b, Sweep sw, SweepSt 
 }
 
 // ------------------------------------------------------------------------------------
-// The staged sweeps with four waves per tile.  Timestamps taken inside the one-wave kernels
+// The staged sweeps with six waves per tile.  Timestamps taken inside the one-wave kernels
 // above (s_memtime at the phase boundaries of every step, 192x96x96 level) split a step of
 // about 4,000 cycles into the face inputs (about 900: LDS reads of the exchange buffers and
 // the halo ring, the marker tests), the recurrence and the three outgoing face
@@ -3015,20 +3016,22 @@ __global__ void __launch_bounds__(TW) k_corr_st(Prm p, Blk b, Sweep sw, SweepSt 
 // * waves 0-2 all form dn of the step from the same inputs, and wave f then forms only the
 //   contribution across face f (0: I, 1: J, 2: K) and leaves it in LDS; wave 1 publishes
 //   the J-face halo words and wave 2 the K-face ones;
-// * wave 3 issues every LDS-DMA copy (records, increments, halo blocks) and waits for them,
-//   so the three compute waves never wait on memory;
+// * waves 3 and 4 issue the LDS-DMA copies (records, increments) and wait for them, wave 5
+//   takes the upstream tiles' halo words, so the three compute waves never wait on memory;
 // * one workgroup barrier per step separates a step's LDS writes from the next step's
-//   reads (the exchange buffers are double-buffered by step parity), and the copy wave
-//   reaches it only once the copies of the next step are complete.
+//   reads (the exchange buffers are double-buffered by step parity), and the other waves
+//   reach it only once what the next step reads is there.
 // Arithmetic is that of k_pred_st / k_corr_st, operation for operation, so the results
 // are the same bit for bit.
 // ------------------------------------------------------------------------------------
 constexpr int SW = 3;              // compute waves per workgroup: one per face
-constexpr int WGW = SW + 1;        // and the copy wave
+constexpr int CW = 2;              // copy waves: half of every record each
+constexpr int WGP = SW + CW + 1;   // waves of the predictor: with the halo wave
+constexpr int WGC = WGP + 1;       // and of the corrector: with the store wave
 
 // The workgroup's exchange point between two steps: LDS writes before it are visible to
 // every wave after it.  Global memory is not ordered (the halo slots carry their own
-// protocol, and the copy wave waits for its LDS-DMA copies with vm_wait before it).
+// protocol, and the copy waves wait for their LDS-DMA copies with vm_wait before it).
 __device__ __forceinline__ void wg_step_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -3044,245 +3047,342 @@ __device__ __forceinline__ int tile_ticket_wg(const Sweep &s, int *slot)
     return __builtin_amdgcn_readfirstlane(*slot);
 }
 
-// PREDGS / PRKEGS on staged records, four waves per (J,K) tile.  The copy wave's issue order
-// within step s: the halo blocks of step s + 2, the record of step s + 3; at the top of step
-// s the two later records (2 NLD loads) follow the halo blocks of step s, which follow the
-// record of step s, so waiting until 2 NLD loads remain covers both.
-template <bool KE, typename RT = double>
-__global__ void __launch_bounds__(WGW * TW) k_pred_wg(Prm p, Blk b, Sweep sw, SweepSt st)
+// PREDGS / PRKEGS (FWD = false) or DIAGGS + CORRGS / DIKEGS + COKEGS with the end of IMPS
+// (FWD = true: DRO/CP, D(rho k) and D(rho omega) times RO) on staged records.
+//
+// What bounds it: a step's latency times the I + J + K - 2 hyperplanes, plus the store-to-load
+// latency of every tile the wavefront crosses.  A step is two phases with a workgroup barrier
+// after each: in the first wave 0 forms the increments dn from its own I-contribution (kept in
+// registers) and the J- and K-contributions of the neighbour columns; in the second waves
+// 0-2 each form the contribution of dn across one face.  The three waves forming dn each for
+// itself needs one barrier less, but then each reads the 21 contributions and the increments'
+// fields from LDS at the same moment, 93 LDS instructions of 1 KiB a step against 62 here,
+// and the LDS becomes what the step waits for.  Everything else is kept off these
+// waves: they read the next record while they would wait (a wave's 15 outstanding LDS
+// instructions are never exceeded), the exchange buffers have a ninth column or row that the
+// halo wave fills with the upstream tile's words (or that stays zero at the block's edge), so
+// that a lane reads its inputs at a constant offset with no test, and the corrector's results
+// go to the fields through LDS in runs of eight cells by a wave of their own (a lane's cell is
+// on a cache line of its own: 64 partial lines per store held up the record copies).
+// Measured (k-omega, FP64 records, predictor / corrector, us; one phase of four waves per tile
+// that read the record after the barrier, tested every halo word and stored to the fields
+// themselves -> this form): 128x64x64 383 / 406 -> 194 / 216, 192x96x96 609 / 643 -> 337 / 378,
+// 48x24x24 130 / 138 -> 72 / 78; one tile of 192 cells takes 0.68 us a step, and crossing a
+// tile costs 8 steps and about 2 us.
+template <bool FWD, bool KE, typename RT = double>
+__global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk b, Sweep sw, SweepSt st)
 {
-    constexpr int NV = KE ? 7 : 5;
-    constexpr int RS = 4;                               // ring slots: 3 steps of lead
+    constexpr int NV = KE ? 7 : 5, NS = KE ? 7 : 4;
+    constexpr bool F32 = sizeof(RT) == 4;
+    constexpr int NW = FWD ? WGC : WGP;
+    constexpr int RS = FWD ? (F32 ? 6 : 3) : (F32 ? 8 : 5);   // ring slots: RS - 1 steps of lead
     constexpr int RBYTES = rbytes<RT>();
-    constexpr int NLD = RBYTES / 1024;                  // record loads per step
-    static_assert(NLD * (RS - 2) <= 63, "vmcnt range");
+    constexpr int NLD = (RBYTES + (FWD ? DBYTES : 0)) / 1024 / CW;   // a copy wave's loads per step
+    static_assert(NLD * (RS - 1) <= 63, "vmcnt range");
+    static_assert(RBYTES / CW % 1024 == 0 && DBYTES / CW % 1024 == 0, "whole loads per copy wave");
+    constexpr int XJ = TJ + 1;                          // row stride of the J exchange buffer
+    constexpr int HST = 4;                              // halo staging slots
+    constexpr int OS = 9, OST = TW + 4;                 // result slots per column, their stride
     __shared__ __attribute__((aligned(16))) RT ring[RS][NRF * TW];
-    __shared__ __attribute__((aligned(16))) double hring[HR][2][HBLK];
-    __shared__ double xo[SW][2][NV][TW], zx[NV * TK];
+    __shared__ __attribute__((aligned(16))) double dring[FWD ? RS : 1][NDN * TW];
+    __shared__ __attribute__((aligned(16))) double hst[HST][2][HBLK];
+    __shared__ double xj[NV][XJ * TK], xk[NV][TJ * (TK + 1)], xd[NV][TW];
+    __shared__ double obuf[FWD ? NV + 1 : 1][FWD ? OS * OST : 1];
     __shared__ int tkt;
-    const RT *const recp = (const RT *)st.recp;
+    const RT *const rec = (const RT *)(FWD ? st.recc : st.recp);
     const int lane = threadIdx.x % TW, w = __builtin_amdgcn_readfirstlane(threadIdx.x / TW);
     const int jj = lane % TJ, kk = lane / TJ;
-    if (w == 0) {
-        if (lane < NV * TK) zx[lane] = 0.;
-        // a lane's I-face input before its first cell is zero
-#pragma unroll
-        for (int r = 0; r < NV; r++) xo[0][0][r][lane] = xo[0][1][r][lane] = 0.;
-    }
-    const int t = tile_ticket_wg(sw, &tkt);
-    const int tj = sw.ntj - 1 - t % sw.ntj, tk = sw.ntk - 1 - t / sw.ntj;
+    // zero: the columns beyond the block's edge
+    for (int q = threadIdx.x; q < NV * XJ * TK; q += NW * TW) (&xj[0][0])[q] = 0.;
+    for (int q = threadIdx.x; q < NV * TJ * (TK + 1); q += NW * TW) (&xk[0][0])[q] = 0.;
+    const int t = tile_ticket_wg(sw, &tkt);             // a workgroup barrier
+    const int tj = FWD ? t % sw.ntj : sw.ntj - 1 - t % sw.ntj;
+    const int tk = FWD ? t / sw.ntj : sw.ntk - 1 - t / sw.ntj;
     const int tile = tk * sw.ntj + tj;
-    const int j = tj * TJ + jj + 1, k = tk * TK + kk + 1;
-    const bool col = j <= b.jmax && k <= b.kmax;
-    const bool hasj = tj + 1 < sw.ntj, hask = tk + 1 < sw.ntk;   // upstream tiles
-    const int lag = (TJ - 1 - jj) + (TK - 1 - kk);
     const int nsteps = st.nstep;
-    const unsigned long long *hj0 = hj_blk(sw, b, tj + 1, tk, 0), *hk0 = hk_blk(sw, b, tk + 1, tj, 0);
-    auto halo_copy = [&](int s) {
-        const int d = b.imax + TK - 2 - s;
-        if (d < 0 || d > b.imax + TK - 2) return;
-        if (hasj) halo_dma(hj0 + (size_t)d * HBLK, hring[s % HR][0], lane);
-        if (hask) halo_dma(hk0 + (size_t)d * HBLK, hring[s % HR][1], lane);
-    };
-    auto rec_copy = [&](int s) {
-        ring_copy<RBYTES>(recp + st_row(st, tile, nsteps - 1 - s, 0), ring[s % RS], lane);
-    };
-    const FaceSrc fj(j == b.jmax, jj < TJ - 1, &xo[1][0][0][min(lane + 1, TW - 1)], hring[0][0] + kk, zx + kk);
-    const FaceSrc fk(k == b.kmax, kk < TK - 1, &xo[2][0][0][min(lane + TJ, TW - 1)], hring[0][1] + jj, zx + jj);
-    const bool copier = w == SW;
-    if (copier) {
-        rec_copy(0);
-        halo_copy(0);
-        if (1 < nsteps) rec_copy(1);
-        halo_copy(1);
-        if (2 < nsteps) rec_copy(2);
-    }
-    for (int s = 0; s < nsteps; s++) {
-        const int row = nsteps - 1 - s;
-        if (copier) {
-            if (s + RS - 2 < nsteps) vm_wait<NLD * (RS - 2)>(); else vm_wait<0>();
-        }
-        wg_step_sync();
-        if (copier) {
-            // the slots of step s - 1, which every wave has finished reading
-            halo_copy(s + 2);
-            if (s + RS - 1 < nsteps) rec_copy(s + RS - 1);
-            continue;
-        }
-        const RT *cur = ring[s % RS] + lane;
-        const int q = s - lag;
-        if (col && q >= 0 && q < b.imax) {
-            const int i = b.imax - q;
-            const int rb = (s + 1) & 1;
-            double yi[NV], bj[NV], ckc[NV];
-#pragma unroll
-            for (int r = 0; r < NV; r++) yi[r] = xo[0][rb][r][lane];
-            const unsigned xoff = rb * (NV * TW * 8), hoff = (s % HR) * (2 * HBLK * 8);
-            faces_in<NV>(fj.at(xoff, hoff), fj.stride, fj.hmask != 0,
-                         [&] { return hj_slot(sw, b, tj + 1, i, k); },
-                         fk.at(xoff, hoff), fk.stride, fk.hmask != 0,
-                         [&] { return hk_slot(sw, b, tk + 1, i, j); }, sw.err, bj, ckc);
-            // the line-buffer shift of PREDGS (imps4.f:556-562) never hands the I+1
-            // contribution to a cell of the row J = JMAX; PRKEGS's (imps4.f:1762) does
-            if (!KE && j == b.jmax) {
-#pragma unroll
-                for (int r = 0; r < NV; r++) yi[r] = 0.;
-            }
-            double dn[NV];
-#pragma unroll
-            for (int r = 0; r < NV; r++) {
-                double cd = cur[RP_MK * TW] * ckc[r] + cur[(RP_VD + r) * TW];
-                cd = cd - cur[RP_DT1 * TW] * (cur[RP_WI * TW] * yi[r] + cur[RP_WJ * TW] * bj[r]);
-                dn[r] = r != 4 ? cd * cur[RP_SCINV * TW] : cd * cur[RP_SCINP * TW];
-            }
-            // the increments for the corrector, their stores dealt between the waves
-            double *dno = st.dn + (((size_t)tile * nsteps + row) * NDN) * TW + lane;
-#pragma unroll
-            for (int r = 0; r < NV; r++)
-                if (r % SW == w) dno[(size_t)r * TW] = dn[r];
-            SweepCell sc;
-            double scv[7];
-#pragma unroll
-            for (int m = 0; m < 7; m++) scv[m] = cur[(RP_SC + m) * TW];
-            sc_get<KE>(sc, scv);
-            double bv[NB];
-#pragma unroll
-            for (int m = 0; m < NB; m++) bv[m] = cur[(RP_N + NB * w + m) * TW];
-            Coef cf;
-            cf.x1 = cur[(RP_X + 3 * w) * TW];
-            cf.x2 = cur[(RP_X + 3 * w + 1) * TW];
-            cf.x5 = cur[(RP_X + 3 * w + 2) * TW];
-            double o[NV];
-            face_xfer<KE>(dn, sc, basis_get(bv), cf, o);
-            const int wb = s & 1;
-#pragma unroll
-            for (int r = 0; r < NV; r++) xo[w][wb][r][lane] = o[r];
-            if (w == 1 && jj == 0 && j > 1) halo_put<NV, HQS>(hj_slot(sw, b, tj, i, k), o);
-            if (w == 2 && kk == 0 && k > 1) halo_put<NV, HQS>(hk_slot(sw, b, tk, i, j), o);
-        }
-    }
-    vm_wait<0>();
-}
+    // the record row of step s: the predictor takes them from the last
+    auto row = [&](int s) { return FWD ? s : nsteps - 1 - s; };
+    // Barriers of every wave: one at the start, two per step (after dn, after the contributions).
 
-// DIAGGS + CORRGS / DIKEGS + COKEGS on staged records, four waves per tile, with the end of
-// IMPS (DRO/CP, D(rho k) and D(rho omega) times RO).  The copy wave's issue order within
-// step s: the halo blocks of step s + 2, the record and increments of step s + 2 (NLD
-// loads); at the top of step s the copy of step s + 1 follows that of step s, which follows
-// the halo blocks of step s, so waiting until NLD loads remain covers both.
-template <bool KE, typename RT = double>
-__global__ void __launch_bounds__(WGW * TW) k_corr_wg(Prm p, Blk b, Sweep sw, SweepSt st)
-{
-    constexpr int NV = KE ? 7 : 5;
-    constexpr int RS = 3;                               // ring slots: 2 steps of lead
-    constexpr int RBYTES = rbytes<RT>();
-    constexpr int NLD = (RBYTES + DBYTES) / 1024;       // record loads per step
-    static_assert(NLD * (RS - 2) <= 63, "vmcnt range");
-    __shared__ __attribute__((aligned(16))) RT ring[RS][NRF * TW];
-    __shared__ __attribute__((aligned(16))) double dring[RS][NDN * TW];
-    __shared__ __attribute__((aligned(16))) double hring[HR][2][HBLK];
-    __shared__ double xo[SW][2][NV][TW], zx[NV * TK];
-    __shared__ int tkt;
-    const RT *const recc = (const RT *)st.recc;
-    const int lane = threadIdx.x % TW, w = __builtin_amdgcn_readfirstlane(threadIdx.x / TW);
-    const int jj = lane % TJ, kk = lane / TJ;
-    if (w == 0) {
-        if (lane < NV * TK) zx[lane] = 0.;
-#pragma unroll
-        for (int r = 0; r < NV; r++) xo[0][0][r][lane] = xo[0][1][r][lane] = 0.;
+    if (w >= SW && w < SW + CW) {
+        // a copy wave.  The last read of record s is in the first phase of step s, the first
+        // one of record s + 1 in the second phase of step s: before the first barrier of step
+        // s record s + 1 must have arrived, of the copies issued by then (up to record
+        // s - 1 + RS) the last RS - 2 may still be in flight, and after it slot s is free.
+        const int c = w - SW;
+        auto copy = [&](int s) {
+            ring_copy<RBYTES / CW>((const char *)(rec + st_row(st, tile, row(s), 0)) + c * (RBYTES / CW),
+                                   (char *)ring[s % RS] + c * (RBYTES / CW), lane);
+            if (FWD)
+                ring_copy<DBYTES / CW>((const char *)(st.dn + (((size_t)tile * nsteps + s) * NDN) * TW) + c * (DBYTES / CW),
+                                       (char *)dring[s % RS] + c * (DBYTES / CW), lane);
+        };
+        for (int s = 0; s < RS && s < nsteps; s++) copy(s);
+        if (RS <= nsteps) vm_wait<NLD * (RS - 1)>(); else vm_wait<0>();
+        wg_step_sync();
+        for (int s = 0; s < nsteps; s++) {
+            if (s - 1 + RS < nsteps) vm_wait<NLD * (RS - 2)>(); else vm_wait<0>();
+            wg_step_sync();
+            if (s + RS < nsteps) copy(s + RS);
+            wg_step_sync();
+        }
+        vm_wait<0>();
+        return;
     }
-    const int t = tile_ticket_wg(sw, &tkt);
-    const int tj = t % sw.ntj, tk = t / sw.ntj;
-    const int tile = tk * sw.ntj + tj;
+
+    if (w == SW + CW) {
+        // the halo wave: lane (word q, offset e along the face) takes word q of the edge
+        // column e from the upstream tile's slots, J and K face alike.  The blocks of a step
+        // are copied to LDS HLEAD steps ahead (so that no step waits for its own loads); words
+        // that were still empty then (either 32-bit half, as a copy may race the store) are
+        // polled.  The values of step s go to the exchange buffers' halo column in the second
+        // phase of step s - 1.  At the end the wave empties the slots it has read for the
+        // next sweep.
+        constexpr int HLEAD = 0;
+        const int e = lane % TK, q = lane / TK, qv = q < NV ? q : 0;
+        const bool inj = q < NV && (FWD ? tj > 0 : tj + 1 < sw.ntj) && tk * TK + e + 1 <= b.kmax;
+        const bool ink = q < NV && (FWD ? tk > 0 : tk + 1 < sw.ntk) && tj * TJ + e + 1 <= b.jmax;
+        unsigned long long *const sj = sw.hj + ((size_t)(FWD ? tj : tj + 1) * sw.ntk + tk) * (b.imax + TK) * HBLK;
+        unsigned long long *const sk = sw.hk + ((size_t)(FWD ? tk : tk + 1) * sw.ntj + tj) * (b.imax + TJ) * HBLK;
+        // the anti-diagonal I + e - 1 of the edge columns' cells at step s
+        auto diag = [&](int s) { return FWD ? s : b.imax + TK - 2 - s; };
+        auto copy = [&](int s) {
+            const size_t d = (size_t)min(max(diag(s), 0), b.imax + TK - 1) * HBLK;
+            halo_dma(sj + d, hst[s % HST][0], lane);
+            halo_dma(sk + d, hst[s % HST][1], lane);
+        };
+        static_assert(HST > HLEAD + 1, "a staging slot is read before it is filled again");
+        const int xjo = e * XJ + (FWD ? 0 : TJ), xko = (FWD ? 0 : TJ * TK) + e;
+        // step s: the copies of the HLEAD later steps have been issued after its own
+        auto take = [&](int s) {
+            const int i = diag(s) - e + 1;
+            const bool live = i >= 1 && i <= b.imax, lj = inj && live, lk = ink && live;
+            vm_wait<2 * HLEAD>();
+            unsigned long long vj = __double_as_longlong(hst[s % HST][0][qv * TK + e]);
+            unsigned long long vk = __double_as_longlong(hst[s % HST][1][qv * TK + e]);
+            bool pj = lj && half_empty(vj), pk = lk && half_empty(vk);
+            if (__builtin_amdgcn_ballot_w64(pj || pk)) {
+                const size_t d = (size_t)(live ? diag(s) : 0) * HBLK + lane;
+                int spins = 0;
+                do {
+                    if ((++spins & 255) == 0) {
+                        if (spins > SPIN_LIMIT) __hip_atomic_fetch_or(sw.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if (spins > SPIN_LIMIT || __hip_atomic_load(sw.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                            if (pj) vj = 0;
+                            if (pk) vk = 0;
+                            break;
+                        }
+                    }
+                    if (pj) vj = __hip_atomic_load(sj + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (pk) vk = __hip_atomic_load(sk + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    pj = pj && vj == HALO_EMPTY;
+                    pk = pk && vk == HALO_EMPTY;
+                } while (__builtin_amdgcn_ballot_w64(pj || pk));
+            }
+            if (lj) xj[qv][xjo] = __longlong_as_double((long long)vj);
+            if (lk) xk[qv][xko] = __longlong_as_double((long long)vk);
+        };
+        for (int m = 0; m <= HLEAD; m++) copy(m);
+        take(0);
+        wg_step_sync();
+        for (int s = 0; s < nsteps; s++) {
+            copy(s + 1 + HLEAD);
+            wg_step_sync();
+            if (s + 1 < nsteps) take(s + 1);
+            wg_step_sync();
+        }
+        vm_wait<0>();
+        for (int d = 0; d < b.imax + TK - 1; d++) {
+            if (inj) __hip_atomic_store(sj + (size_t)d * HBLK + lane, HALO_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (ink) __hip_atomic_store(sk + (size_t)d * HBLK + lane, HALO_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        return;
+    }
+
     const int j = tj * TJ + jj + 1, k = tk * TK + kk + 1;
     const bool col = j <= b.jmax && k <= b.kmax;
-    const bool hasj = tj > 0, hask = tk > 0;                  // upstream tiles
-    const int lag = jj + kk;
-    const int nsteps = st.nstep;
-    const unsigned long long *hj0 = hj_blk(sw, b, tj, tk, 0), *hk0 = hk_blk(sw, b, tk, tj, 0);
-    auto halo_copy = [&](int s) {
-        if (s > b.imax + TK - 2) return;
-        if (hasj) halo_dma(hj0 + (size_t)s * HBLK, hring[s % HR][0], lane);
-        if (hask) halo_dma(hk0 + (size_t)s * HBLK, hring[s % HR][1], lane);
-    };
-    const FaceSrc fj(j == 1, jj > 0, &xo[1][0][0][max(lane - 1, 0)], hring[0][0] + kk, zx + kk);
-    const FaceSrc fk(k == 1, kk > 0, &xo[2][0][0][max(lane - TJ, 0)], hring[0][1] + jj, zx + jj);
-    auto rec_copy = [&](int s) {
-        ring_copy<RBYTES>(recc + st_row(st, tile, s, 0), ring[s % RS], lane);
-        ring_copy<DBYTES>(st.dn + (((size_t)tile * nsteps + s) * NDN) * TW, dring[s % RS], lane);
-    };
-    const bool copier = w == SW;
-    if (copier) {
-        halo_copy(0);
-        rec_copy(0);
-        halo_copy(1);
-        if (1 < nsteps) rec_copy(1);
-    }
-    for (int s = 0; s < nsteps; s++) {
-        if (copier) {
-            if (s + RS - 2 < nsteps) vm_wait<NLD * (RS - 2)>(); else vm_wait<0>();
-        }
+    const int lag = FWD ? jj + kk : (TJ - 1 - jj) + (TK - 1 - kk);
+    double *out[NV];
+#pragma unroll
+    for (int m = 0; m < NV; m++) out[m] = FLD(b, FF_DRO + m);
+
+    if (FWD && w == SW + CW + 1) {
+        // the store wave.  Column (jj, kk) leaves its cell q = s - jj - kk of step s in slot
+        // q % OS.  After the steps with s - jj - kk = 7 (mod 8) a run of eight cells is
+        // complete: one column for every jj.  Lane (c, m) stores cell m of the run of column
+        // jj = c in the first phase of the next step but one; the cell written meanwhile has a
+        // slot of its own.  DRO/CP is formed here, off the compute waves.
+        const int c = lane / 8, m8 = lane % 8;
+        auto store = [&](int s) {
+            const int ck = (s + 1 - c) & 7, q = s - c - ck - 7 + m8;
+            const int cj = tj * TJ + c + 1, ckk = tk * TK + ck + 1;
+            if (q < 0 || q >= b.imax || cj > b.jmax || ckk > b.kmax) return;
+            const int o = (q % OS) * OST + ck * TJ + c, n = cid(b, q + 1, cj, ckk);
+#pragma unroll
+            for (int m = 1; m < NV; m++) out[m][n] = obuf[m][o];
+            out[0][n] = obuf[0][o] / obuf[NV][o];
+        };
         wg_step_sync();
-        if (copier) {
-            halo_copy(s + 2);
-            if (s + RS - 1 < nsteps) rec_copy(s + RS - 1);
-            continue;
+        for (int s = 0; s < nsteps; s++) {
+            store(s - 1);
+            wg_step_sync();
+            wg_step_sync();
         }
-        const RT *cur = ring[s % RS] + lane;
-        const double *dni = dring[s % RS] + lane;
-        const int q = s - lag;
-        if (col && q >= 0 && q < b.imax) {
-            const int i = q + 1;
-            const int n = cid(b, i, j, k);
-            const int rb = (s + 1) & 1;
-            double yi[NV], bj[NV], ckc[NV];
-#pragma unroll
-            for (int r = 0; r < NV; r++) yi[r] = xo[0][rb][r][lane];
-            const unsigned xoff = rb * (NV * TW * 8), hoff = (s % HR) * (2 * HBLK * 8);
-            faces_in<NV>(fj.at(xoff, hoff), fj.stride, fj.hmask != 0,
-                         [&] { return hj_slot(sw, b, tj, i, k); },
-                         fk.at(xoff, hoff), fk.stride, fk.hmask != 0,
-                         [&] { return hk_slot(sw, b, tk, i, j); }, sw.err, bj, ckc);
-            double d[NV];
-#pragma unroll
-            for (int r = 0; r < NV; r++) d[r] = dni[r * TW] * cur[RC_FAC * TW];
-            double dn[NV];
-#pragma unroll
-            for (int r = 0; r < NV; r++) {
-                double cd = cur[RC_MK * TW] * ckc[r] + cur[RC_VOL * TW] * d[r];
-                cd = cd + cur[RC_DT1 * TW] * (cur[RC_WI * TW] * yi[r] + cur[RC_WJ * TW] * bj[r]);
-                dn[r] = r != 4 ? cd * cur[RC_SCINV * TW] : cd * cur[RC_SCINP * TW];
-            }
-            // the end of IMPS, its stores dealt between the waves
-            if (w == 0) FLD(b, FF_DRO)[n] = dn[0] / cur[RC_CP * TW];
-#pragma unroll
-            for (int r = 1; r < 5; r++)
-                if (r % SW == w) FLD(b, FF_DRO + r)[n] = dn[r];
-            if (KE) {
-                if (w == 2) FLD(b, FF_DRK)[n] = dn[NV > 5 ? 5 : 0] * cur[RC_RHO * TW];
-                if (w == 0) FLD(b, FF_DEPS)[n] = dn[NV > 6 ? 6 : 0] * cur[RC_RHO * TW];
-            }
-            SweepCell sc;
-            double scv[7];
-#pragma unroll
-            for (int m = 0; m < 7; m++) scv[m] = cur[(RC_SC + m) * TW];
-            sc_get<KE>(sc, scv);
-            double bv[NB];
-#pragma unroll
-            for (int m = 0; m < NB; m++) bv[m] = cur[(RC_N + NB * w + m) * TW];
-            Coef cf;
-            cf.x1 = cur[(RC_X + 3 * w) * TW];
-            cf.x2 = cur[(RC_X + 3 * w + 1) * TW];
-            cf.x5 = cur[(RC_X + 3 * w + 2) * TW];
-            double o[NV];
-            face_xfer<KE>(dn, sc, basis_get(bv), cf, o);
-            const int wb = s & 1;
-#pragma unroll
-            for (int r = 0; r < NV; r++) xo[w][wb][r][lane] = o[r];
-            if (w == 1 && jj == TJ - 1 && j < b.jmax) halo_put<NV, HQS>(hj_slot(sw, b, tj + 1, i, k), o);
-            if (w == 2 && kk == TK - 1 && k < b.kmax) halo_put<NV, HQS>(hk_slot(sw, b, tk + 1, i, j), o);
-        }
+        for (int s = nsteps - 1; s < nsteps + 8; s++) store(s);
+        return;
     }
-    vm_wait<0>();
+
+    auto compute = [&](auto wave) __attribute__((always_inline)) {
+        constexpr int W = decltype(wave)::value;
+        // where this lane's contribution goes and where wave 0 finds its neighbours'
+        const int wj = FWD ? kk * XJ + jj + 1 : kk * XJ + jj, rj = FWD ? wj - 1 : wj + 1;
+        const int wk = FWD ? lane + TJ : lane, rk = FWD ? wk - TJ : wk + TJ;
+        // this wave's outgoing halo words: J-faces from wave 1, K-faces from wave 2
+        const bool put = W == 1 ? (FWD ? jj == TJ - 1 && j < b.jmax : jj == 0 && j > 1)
+                                : W == 2 && (FWD ? kk == TK - 1 && k < b.kmax : kk == 0 && k > 1);
+        unsigned long long *const pslot =
+            W == 1 ? sw.hj + ((size_t)(FWD ? tj + 1 : tj) * sw.ntk + tk) * (b.imax + TK) * HBLK + kk
+                   : sw.hk + ((size_t)(FWD ? tk + 1 : tk) * sw.ntj + tj) * (b.imax + TJ) * HBLK + jj;
+        // the line-buffer shift of PREDGS (imps4.f:556-562) never hands the I+1 contribution to
+        // a cell of the row J = JMAX; PRKEGS's (imps4.f:1762) does
+        const bool noi = !FWD && !KE && j == b.jmax;
+        // wave 0: the increments' fields of a record, with VOL times the increments
+        RT vd[NV], mk, dt1, wi, wjj, scinv, scinp, fac, vol;
+        double dni[NV], cd[NV], yi[NV];
+        auto read_dn = [&](const RT *r, const double *d) __attribute__((always_inline)) {
+            if (FWD) {
+#pragma unroll
+                for (int m = 0; m < NV; m++) dni[m] = d[m * TW];
+                fac = r[RC_FAC * TW]; vol = r[RC_VOL * TW];
+            } else {
+#pragma unroll
+                for (int m = 0; m < NV; m++) vd[m] = r[(RP_VD + m) * TW];
+            }
+            mk = r[(FWD ? RC_MK : RP_MK) * TW]; dt1 = r[(FWD ? RC_DT1 : RP_DT1) * TW];
+            wi = r[(FWD ? RC_WI : RP_WI) * TW]; wjj = r[(FWD ? RC_WJ : RP_WJ) * TW];
+            scinv = r[(FWD ? RC_SCINV : RP_SCINV) * TW]; scinp = r[(FWD ? RC_SCINP : RP_SCINP) * TW];
+        };
+        auto vol_dn = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int m = 0; m < NV; m++) cd[m] = FWD ? vol * (dni[m] * fac) : (double)vd[m];
+        };
+#pragma unroll
+        for (int m = 0; m < NV; m++) yi[m] = 0.;          // before a lane's first cell
+        int slot = 0, os = 0;
+        wg_step_sync();
+        if (W == 0) {
+            read_dn(ring[0] + lane, dring[0] + lane);
+            vol_dn();
+        }
+        for (int s = 0; s < nsteps; s++) {
+            const RT *const rc = ring[slot] + lane;
+            slot = slot + 1 == RS ? 0 : slot + 1;
+            const int q = s - lag;
+            const bool act = col && q >= 0 && q < b.imax;
+            const int i = FWD ? q + 1 : b.imax - q;
+            double dn[NV], bj[NV], ck[NV];
+            RT sv[NS], bs[NB], xs[3], aux;
+            // ---- first phase: dn ------------------------------------------------------
+            if (W == 0) {
+#pragma unroll
+                for (int m = 0; m < NV; m++) {
+                    ck[m] = xk[m][rk];
+                    bj[m] = xj[m][rj];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the face's fields: waves 1 and 2 read them behind wave 0's inputs, which the
+            // step waits for, wave 0 its own in the second phase
+            auto read_face = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int m = 0; m < NS; m++) sv[m] = rc[((FWD ? RC_SC : RP_SC) + m) * TW];
+#pragma unroll
+                for (int m = 0; m < NB; m++) bs[m] = rc[((FWD ? RC_N : RP_N) + W * NB + m) * TW];
+#pragma unroll
+                for (int m = 0; m < 3; m++) xs[m] = rc[((FWD ? RC_X : RP_X) + W * 3 + m) * TW];
+                if (FWD) aux = rc[(W == 0 ? RC_CP : RC_RHO) * TW];
+            };
+            if (W > 0) {
+                __builtin_amdgcn_s_sleep(4);
+                read_face();
+            }
+            if (W == 0) {
+                double wy[NV];
+#pragma unroll
+                for (int m = 0; m < NV; m++) wy[m] = wi * (noi ? 0. : yi[m]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int m = 0; m < NV; m++) {
+                    double c = mk * ck[m] + cd[m];
+                    const double d = dt1 * (wy[m] + wjj * bj[m]);
+                    c = FWD ? c + d : c - d;
+                    dn[m] = m != 4 ? c * scinv : c * scinp;
+                }
+#pragma unroll
+                for (int m = 0; m < NV; m++) xd[m][lane] = dn[m];
+            }
+            double bv[NB];
+            FaceBasis fb;
+            auto basis = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int m = 0; m < NB; m++) bv[m] = bs[m];
+                fb = basis_get(bv);
+            };
+            if (W > 0) basis();
+            wg_step_sync();
+            // ---- second phase: the contribution across face W --------------------------
+            if (W > 0) {
+#pragma unroll
+                for (int m = 0; m < NV; m++) dn[m] = xd[m][lane];
+            } else {
+                read_face();
+                __builtin_amdgcn_sched_barrier(0);
+                basis();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            SweepCell sc;
+            double scv[7], o[NV];
+#pragma unroll
+            for (int m = 0; m < NS; m++) scv[m] = sv[m];
+            sc_get<KE>(sc, scv);
+            Coef cf;
+            cf.x1 = xs[0]; cf.x2 = xs[1]; cf.x5 = xs[2];
+            if (act) {
+                face_xfer<KE>(dn, sc, fb, cf, o);
+#pragma unroll
+                for (int m = 0; m < NV; m++) {
+                    if (W == 0) yi[m] = o[m];
+                    else if (W == 1) xj[m][wj] = o[m];
+                    else xk[m][wk] = o[m];
+                }
+                if (W > 0 && put) halo_put<NV, HQS>(pslot + (size_t)(i + (W == 1 ? kk : jj) - 1) * HBLK, o);
+                // the increments (for the corrector) or the end of IMPS, dealt between the waves
+                if (!FWD) {
+                    double *dno = st.dn + (((size_t)tile * nsteps + row(s)) * NDN) * TW + lane;
+#pragma unroll
+                    for (int m = 0; m < NV; m++)
+                        if (m % SW == W) dno[(size_t)m * TW] = dn[m];
+                } else {
+                    const int ob = os * OST + lane;
+#pragma unroll
+                    for (int m = 0; m < 5; m++)
+                        if (m % SW == W) obuf[m][ob] = dn[m];
+                    if (W == 0) obuf[NV][ob] = aux;
+                    if (KE && W == 2) obuf[NV > 5 ? 5 : 0][ob] = dn[NV > 5 ? 5 : 0] * aux;
+                    if (KE && W == 1) obuf[NV > 6 ? 6 : 0][ob] = dn[NV > 6 ? 6 : 0] * aux;
+                }
+            }
+            if (FWD && q >= 0) os = os + 1 == OS ? 0 : os + 1;
+            if (W == 0) {
+                read_dn(ring[slot] + lane, dring[FWD ? slot : 0] + lane);
+                vol_dn();
+            }
+            wg_step_sync();
+        }
+    };
+    if (w == 0) compute(std::integral_constant<int, 0>());
+    else if (w == 1) compute(std::integral_constant<int, 1>());
+    else compute(std::integral_constant<int, 2>());
 }
 
 // ------------------------------------------------------------------------------------
@@ -4945,29 +5045,31 @@ static int implicit_impl(ff_ctx *c, BlockRec *r, int level, bool divcp)
         const bool f32 = c->precision == FF_PREC_MIXED;
         auto prep = ke ? (f32 ? k_sweep_prep<true, float> : k_sweep_prep<true>)
                        : (f32 ? k_sweep_prep<false, float> : k_sweep_prep<false>);
-        // FF_LUSGS_STAGED: four waves per tile; FF_LUSGS_STAGED1: one
+        // FF_LUSGS_STAGED: six waves per tile; FF_LUSGS_STAGED1: one
         const bool w1 = c->lusgs_mode == FF_LUSGS_STAGED1;
         auto pred = w1 ? (ke ? (f32 ? k_pred_st<true, float> : k_pred_st<true>)
                              : (f32 ? k_pred_st<false, float> : k_pred_st<false>))
-                       : (ke ? (f32 ? k_pred_wg<true, float> : k_pred_wg<true>)
-                             : (f32 ? k_pred_wg<false, float> : k_pred_wg<false>));
+                       : (ke ? (f32 ? k_sweep_wg<false, true, float> : k_sweep_wg<false, true>)
+                             : (f32 ? k_sweep_wg<false, false, float> : k_sweep_wg<false, false>));
         auto corr = w1 ? (ke ? (f32 ? k_corr_st<true, float> : k_corr_st<true>)
                              : (f32 ? k_corr_st<false, float> : k_corr_st<false>))
-                       : (ke ? (f32 ? k_corr_wg<true, float> : k_corr_wg<true>)
-                             : (f32 ? k_corr_wg<false, float> : k_corr_wg<false>));
-        const dim3 ts(w1 ? TW : WGW * TW);
+                       : (ke ? (f32 ? k_sweep_wg<true, true, float> : k_sweep_wg<true, true>)
+                             : (f32 ? k_sweep_wg<true, false, float> : k_sweep_wg<true, false>));
+        const dim3 tpred(w1 ? TW : WGP * TW), tcorr(w1 ? TW : WGC * TW);
         // (forming the corrector's records on a side stream during the predictor's wavefront
         // was measured slower: the latency-bound sweep loses more than the pass gains)
         rc = launch(c, "k_sweep_prep", prep, gp, dim3(PSW * TW), kp, b, r->sw, r->st, tp);
         if (rc) return rc;
-        // each sweep leaves its halo slots filled; empty them for the next one
+        // the one-wave sweeps leave their halo slots filled: empty them for the next one
         const dim3 gf((unsigned)((r->ntile_slots + 255) / 256));
-        rc = launch(c, "k_pred_st", pred, g, ts, kp, b, r->sw, r->st);
-        if (rc) return rc;
-        if ((rc = launch(c, "k_fill_slots", k_fill_u64, gf, dim3(256), r->sw.hj, r->ntile_slots, HALO_EMPTY))) return rc;
-        rc = launch(c, "k_corr_st", corr, g, ts, kp, b, r->sw, r->st);
-        if (rc) return rc;
-        return launch(c, "k_fill_slots", k_fill_u64, gf, dim3(256), r->sw.hj, r->ntile_slots, HALO_EMPTY);
+        auto empty = [&]() {
+            return w1 ? launch(c, "k_fill_slots", k_fill_u64, gf, dim3(256), r->sw.hj, r->ntile_slots, HALO_EMPTY)
+                      : FF_OK;
+        };
+        if ((rc = launch(c, "k_pred_st", pred, g, tpred, kp, b, r->sw, r->st)) || (rc = empty()) ||
+            (rc = launch(c, "k_corr_st", corr, g, tcorr, kp, b, r->sw, r->st)))
+            return rc;
+        return empty();
     }
     if (c->lusgs_mode == FF_LUSGS_TILES) {
         // DRO/CP is applied inside the forward sweep
