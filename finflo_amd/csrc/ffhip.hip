@@ -3997,10 +3997,10 @@ struct MlpRec {
     float *p = nullptr, *m = nullptr, *v = nullptr;    // parameters and Adam moments
     float *nrm = nullptr;                               // normalisation block
     double *nscr = nullptr;                             // normalisation passes: partials, means
-    float *part = nullptr;                              // per-wave gradient partials
-    unsigned *idx = nullptr;                            // minibatch indices
+    float *part = nullptr;                              // per-workgroup gradient partials
+    float *loss = nullptr;                              // losses of the steps of a training call
     float *grad = nullptr;                              // reduced gradient and loss
-    int part_waves = 0, idx_cap = 0;
+    int parts = 0, loss_cap = 0;
     int step = 0;                                       // Adam steps taken
     bool ready = false;                                 // parameters and normalisation set
 };

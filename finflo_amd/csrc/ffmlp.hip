@@ -26,7 +26,7 @@ constexpr int MOFF_W1 = 0, MOFF_B1 = MOFF_W1 + MNH * MNIN, MOFF_W2 = MOFF_B1 + M
               MOFF_B2 = MOFF_W2 + MNH * MNH, MOFF_W3 = MOFF_B2 + MNH,
               MOFF_B3 = MOFF_W3 + MNOUT * MNH, MNP = MOFF_B3 + MNOUT;
 static_assert(MNP == FF_MLP_NPARAM, "parameter count of the header");
-constexpr int MPP = MNP + 1;           // per-wave partial: gradient, then the loss
+constexpr int MPP = MNP + 1;           // per-workgroup partial: gradient, then the loss
 // normalisation block: x mean (5), x scale (5), y mean (3), y scale (3), hull low (5), high (5)
 constexpr int MN_XM = 0, MN_XS = 5, MN_YM = 10, MN_YS = 13, MN_LO = 16, MN_HI = 21;
 static_assert(MN_HI + 5 == FF_MLP_NNORM, "normalisation block of the header");
@@ -83,35 +83,47 @@ struct MlpFrags {
     float b1[4][4], b2[4][4], b3[4];          // this lane's rows of the biases
 };
 
-__device__ __forceinline__ void mlp_load_frags(const float *p, int lane, MlpFrags &f, bool bwd)
+// The parameters in LDS: the rows of W2 are padded to 65 floats, so that the 16 rows of an
+// operand lie in different banks.  Every wave gathers about 200 values from there; gathered
+// from global memory they were most of a short kernel's time (k_mlp_grad, k_earsm_mlp).
+constexpr int LW2S = MNH + 1, LSH = MNH;              // W2's row stride, the shift behind W2
+constexpr int MLP_LW = MNP + LSH;
+__device__ __forceinline__ void mlp_stage(const float *p, float *w)
+{
+    for (int i = threadIdx.x; i < MNP; i += blockDim.x)
+        w[i < MOFF_W2 ? i : i < MOFF_B2 ? i + (i - MOFF_W2) / MNH : i + LSH] = p[i];
+}
+
+// operands from the staged parameters w
+__device__ __forceinline__ void mlp_load_frags(const float *w, int lane, MlpFrags &f, bool bwd)
 {
     const int g = lane >> 4, c = lane & 15;
 #pragma unroll
-    for (int i = 0; i < 4; i++) f.b3[i] = 4 * g + i < MNOUT ? p[MOFF_B3 + 4 * g + i] : 0.f;
+    for (int i = 0; i < 4; i++) f.b3[i] = 4 * g + i < MNOUT ? w[LSH + MOFF_B3 + 4 * g + i] : 0.f;
 #pragma unroll
     for (int ob = 0; ob < 4; ob++) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int k = 4 * g + i;
-            f.b1[ob][i] = p[MOFF_B1 + 16 * ob + k];
-            f.b2[ob][i] = p[MOFF_B2 + 16 * ob + k];
-            f.w1[ob][i] = bf16_bits(k < MNIN ? p[MOFF_W1 + (16 * ob + c) * MNIN + k] : 0.f);
-            if (bwd) f.w3t[ob][i] = bf16_bits(k < MNOUT ? p[MOFF_W3 + k * MNH + 16 * ob + c] : 0.f);
+            f.b1[ob][i] = w[MOFF_B1 + 16 * ob + k];
+            f.b2[ob][i] = w[LSH + MOFF_B2 + 16 * ob + k];
+            f.w1[ob][i] = bf16_bits(k < MNIN ? w[MOFF_W1 + (16 * ob + c) * MNIN + k] : 0.f);
+            if (bwd) f.w3t[ob][i] = bf16_bits(k < MNOUT ? w[LSH + MOFF_W3 + k * MNH + 16 * ob + c] : 0.f);
         }
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 const int k = phi(kb, g, j);
-                f.w2[ob][kb][j] = bf16_bits(p[MOFF_W2 + (16 * ob + c) * MNH + k]);
-                if (bwd) f.w2t[ob][kb][j] = bf16_bits(p[MOFF_W2 + k * MNH + 16 * ob + c]);
+                f.w2[ob][kb][j] = bf16_bits(w[MOFF_W2 + (16 * ob + c) * LW2S + k]);
+                if (bwd) f.w2t[ob][kb][j] = bf16_bits(w[MOFF_W2 + k * LW2S + 16 * ob + c]);
             }
     }
 #pragma unroll
     for (int kb = 0; kb < 2; kb++)
 #pragma unroll
         for (int j = 0; j < 8; j++)
-            f.w3[kb][j] = bf16_bits(c < MNOUT ? p[MOFF_W3 + c * MNH + phi(kb, g, j)] : 0.f);
+            f.w3[kb][j] = bf16_bits(c < MNOUT ? w[LSH + MOFF_W3 + c * MNH + phi(kb, g, j)] : 0.f);
 }
 
 // Forward pass of 16 cells.  xn: this lane's normalised inputs 4g..4g+3 of cell lane%16.
@@ -185,25 +197,52 @@ __device__ __forceinline__ void mlp_inputs(const float *x, const float *nrm, int
     }
 }
 
-// Inference on samples: physical outputs (beta4, beta6, beta9) of n cells.  Wave w takes
-// cells 16 w .. 16 w + 15 in steps of the grid.
+// orders one wave's LDS writes before its reads of other lanes' values
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Inference on samples: physical outputs (beta4, beta6, beta9) of n cells, 64 cells per wave
+// and pass: a lane transforms its own cell's five inputs and three outputs, and LDS hands
+// them to the four 16-cell passes of the network.  Bound by the exponentials and reciprocals
+// of the 128 activations per cell; transforming the inputs inside every 16-cell pass, where
+// 80 of 256 lane slots hold one, took 343 us on 4.2 M cells against 230.
 __global__ void __launch_bounds__(256) k_mlp_infer(const float *p, const float *nrm, const float *x,
                                                    float *y, int n)
 {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    __shared__ float wts[MLP_LW], xs[4][64][MNIN], ys[4][64][MNOUT];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+    mlp_stage(p, wts);
+    __syncthreads();
     MlpFrags f;
-    mlp_load_frags(p, lane, f, false);
-    const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int nw = gridDim.x * (blockDim.x >> 6);
-    for (int base = 16 * wave; base < n; base += 16 * nw) {
-        const int cell = base + c;
-        float xn[4];
-        mlp_inputs(x, nrm, cell, cell < n, g, xn);
-        MlpFwd o;
-        mlp_forward16(f, lane, xn, o);
-        if (g == 0 && cell < n)
+    mlp_load_frags(wts, lane, f, false);
+    const int nw = gridDim.x * 4;
+    for (long long base = 64ll * (blockIdx.x * 4 + w); base < n; base += 64ll * nw) {
+        const long long cell = base + lane;
+        const bool ok = cell < n;
 #pragma unroll
-            for (int i = 0; i < MNOUT; i++) y[(size_t)cell * MNOUT + i] = mlp_output(o.y[i], nrm, i);
+        for (int q = 0; q < MNIN; q++)
+            xs[w][lane][q] = ok ? (mlp_feature(x[cell * MNIN + q]) - nrm[MN_XM + q]) / nrm[MN_XS + q] : 0.f;
+        wave_lds_sync();
+#pragma unroll 1
+        for (int cb = 0; cb < 4; cb++) {
+            float xn[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) xn[i] = 4 * g + i < MNIN ? xs[w][16 * cb + c][4 * g + i] : 0.f;
+            MlpFwd o;
+            mlp_forward16(f, lane, xn, o);
+            if (g == 0)
+#pragma unroll
+                for (int i = 0; i < MNOUT; i++) ys[w][16 * cb + c][i] = o.y[i];
+        }
+        wave_lds_sync();
+        if (ok)
+#pragma unroll
+            for (int i = 0; i < MNOUT; i++) y[cell * MNOUT + i] = mlp_output(ys[w][lane][i], nrm, i);
+        wave_lds_sync();
     }
 }
 
@@ -233,19 +272,36 @@ __device__ __forceinline__ float xor_sum16(float v)
     return v;
 }
 
-// Loss and gradient partials over a set of samples.  Sample s of the set is sample
-// idx[s] when idx is given, else s.  The loss is the mean over `ntot` samples of the squared
-// error of the normalised outputs summed over the outputs.  Each wave writes its partial
-// gradient and loss to part[wave * MPP ..].
+// Minibatch sample of slot s: a hash of (seed, step, slot), uniform over [0, n)
+struct MlpBatch { int n, step; unsigned seed; };      // n = 0: the samples in order
+__device__ __forceinline__ int mlp_pick(const MlpBatch &bt, int s)
+{
+    unsigned long long h = ((unsigned long long)bt.seed << 32) ^ ((unsigned long long)bt.step * 0x9E3779B97F4A7C15ull) ^ (unsigned long long)s;
+    h ^= h >> 33; h *= 0xFF51AFD7ED558CCDull; h ^= h >> 33; h *= 0xC4CEB9FE1A85EC53ull; h ^= h >> 33;
+    return (int)(h % (unsigned long long)bt.n);
+}
+
+// Loss and gradient partials over a set of samples: all of them or a minibatch.  The loss is
+// the mean over `ntot` samples of the squared error of the normalised outputs summed over
+// the outputs.  The workgroup's four waves are added in order through LDS and it writes its
+// partial gradient and loss to part[blockIdx.x * MPP ..]: a quarter of the partials to sum.
+// A minibatch is latency: the weights' gathers, one pass of 16 samples, the transposes and the
+// sum of the waves.  8192 samples: 38.6 us with gathers from global memory, four passes per
+// wave and a partial per wave; 45.5 with one pass and the waves added to one LDS buffer in
+// turn; 21.4 with the parameters staged in LDS and a buffer per wave.
 __global__ void __launch_bounds__(256) k_mlp_grad(const float *p, const float *nrm, const float *x,
-                                                  const float *t, const unsigned *idx, int nset,
+                                                  const float *t, MlpBatch bt, int nset,
                                                   float inv_ntot, float *part)
 {
-    __shared__ MlpLds lds_all[4];
+    // the staged parameters, the transposes and the waves' sums, one after the other
+    __shared__ union { float w[MLP_LW]; MlpLds t[4]; float sum[4][MPP]; } lds;
     const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    MlpLds &L = lds_all[threadIdx.x >> 6];
+    MlpLds &L = lds.t[threadIdx.x >> 6];
+    mlp_stage(p, lds.w);
+    __syncthreads();
     MlpFrags f;
-    mlp_load_frags(p, lane, f, true);
+    mlp_load_frags(lds.w, lane, f, true);
+    __syncthreads();
     const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int nw = gridDim.x * (blockDim.x >> 6);
     v4f gw1[4], gw2[4][4], gw3[4];
@@ -265,7 +321,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float *p, const float *n
     for (int base = 16 * wave; base < nset; base += 16 * nw) {
         const int s = base + c;
         const bool ok = s < nset;
-        const int cell = ok ? (idx ? (int)idx[s] : s) : 0;
+        const int cell = ok ? (bt.n ? mlp_pick(bt, s) : s) : 0;
         float xn[4];
         mlp_inputs(x, nrm, cell, ok, g, xn);
         MlpFwd o;
@@ -339,8 +395,12 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float *p, const float *n
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     }
-    // partials: weight blocks lane by lane, biases summed over the 16 cell lanes
-    float *o = part + (size_t)wave * MPP;
+    // partials: weight blocks lane by lane, biases summed over the 16 cell lanes, wave after wave
+    float l = loss;
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) l += __shfl_xor(l, m, 64);
+    __syncthreads();
+    float *const o = lds.sum[threadIdx.x >> 6];
 #pragma unroll
     for (int ob = 0; ob < 4; ob++)
 #pragma unroll
@@ -361,22 +421,39 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const float *p, const float *n
         const float s3 = xor_sum16(gb3[i]);
         if (c == 0 && 4 * g + i < MNOUT) o[MOFF_B3 + 4 * g + i] = s3;
     }
-    float l = loss;
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) l += __shfl_xor(l, m, 64);
     if (lane == 0) o[MNP] = l * inv_ntot;
+    __syncthreads();
+    for (int q = threadIdx.x; q < MPP; q += 256)
+        part[(size_t)blockIdx.x * MPP + q] = ((lds.sum[0][q] + lds.sum[1][q]) + lds.sum[2][q]) + lds.sum[3][q];
 }
 
-// Sum of the wave partials in a fixed order; with lr > 0 one Adam step on the parameters
-// (beta1 0.9, beta2 0.999, eps 1e-8; bias-corrected with step number `step` >= 1)
-__global__ void __launch_bounds__(256) k_mlp_reduce(float *p, float *m, float *v, const float *part,
-                                                    int nwave, float lr, int step, float *grad)
+// Sum of the workgroups' partials in a fixed order; with lr > 0 one Adam step on the
+// parameters (beta1 0.9, beta2 0.999, eps 1e-8; bias-corrected with step number `step` >= 1);
+// the loss also to *loss.  16 columns by 16 slices of the partials per workgroup, added as a
+// tree: one thread per column ran through all partials alone, 31.6 us for 128 of them
+// against 4.8 us.
+constexpr int MLP_GRID = 1024;         // workgroups of the looping kernels: four per CU
+constexpr int RDC = 16, RDS = 16;
+__global__ void __launch_bounds__(RDC * RDS) k_mlp_reduce(float *p, float *m, float *v, const float *part,
+                                                          int nparts, float lr, int step, float *grad,
+                                                          float *loss)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= MPP) return;
+    __shared__ float sh[RDS][RDC];
+    const int c = threadIdx.x % RDC, k = threadIdx.x / RDC, j = blockIdx.x * RDC + c;
     float s = 0.f;
-    for (int w = 0; w < nwave; w++) s += part[(size_t)w * MPP + j];
-    if (grad) grad[j] = s;
+    if (j < MPP)
+#pragma unroll 8
+        for (int w = k; w < nparts; w += RDS) s += part[(size_t)w * MPP + j];
+    sh[k][c] = s;
+    __syncthreads();
+    for (int h = RDS / 2; h > 0; h >>= 1) {
+        if (k < h) sh[k][c] += sh[k + h][c];
+        __syncthreads();
+    }
+    if (k || j >= MPP) return;
+    s = sh[0][c];
+    grad[j] = s;
+    if (loss && j == MNP) *loss = s;
     if (lr > 0.f && j < MNP) {
         const float b1 = 0.9f, b2 = 0.999f;
         const float mj = b1 * m[j] + (1.f - b1) * s;
@@ -386,16 +463,6 @@ __global__ void __launch_bounds__(256) k_mlp_reduce(float *p, float *m, float *v
         const float mh = mj / (1.f - powf(b1, (float)step)), vh = vj / (1.f - powf(b2, (float)step));
         p[j] -= lr * mh / (sqrtf(vh) + 1e-8f);
     }
-}
-
-// Minibatch indices: a hash of (seed, step, slot), uniform over [0, n)
-__global__ void __launch_bounds__(256) k_mlp_batch(unsigned *idx, int nb, int n, unsigned seed, int step)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nb) return;
-    unsigned long long h = ((unsigned long long)seed << 32) ^ ((unsigned long long)step * 0x9E3779B97F4A7C15ull) ^ (unsigned long long)s;
-    h ^= h >> 33; h *= 0xFF51AFD7ED558CCDull; h ^= h >> 33; h *= 0xC4CEB9FE1A85EC53ull; h ^= h >> 33;
-    idx[s] = (unsigned)(h % (unsigned long long)n);
 }
 
 // Normalisation block from samples: means and standard deviations of the transformed inputs
@@ -532,61 +599,77 @@ __global__ void __launch_bounds__(256) k_earsm_samples(Blk b, float *x, float *y
 // correction, and the four betas from N by EARSM1's own formulas (earsm.f:196-205), so that
 // they stay consistent with each other (b_ij is a sum of cancelling terms); any other cell
 // takes the exact EARSM1.  Cells are numbered I fastest over the interior.
-__global__ void __launch_bounds__(256) k_earsm_mlp(Blk b, const float *p, const float *nrm)
+// A workgroup loops over 256-cell chunks (the grid fills the chip), so that the parameters
+// are staged and gathered once and not per chunk; at most 256 registers, two waves per SIMD
+// (the exact branch alone would take 280).  256x128x128 cells: 610 us with the parameters
+// gathered per 256 cells, 451 with the loop, 436 with the terms formed twice, 340 with two
+// waves per SIMD.
+__global__ void __launch_bounds__(256, 2) k_earsm_mlp(Blk b, const float *p, const float *nrm)
 {
-    __shared__ float xs[4][64][MNIN];
-    __shared__ float ys[4][64][MNOUT];
+    __shared__ float wts[MLP_LW], xs[4][64][MNIN], ys[4][64][MNOUT];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
     const int ncell = b.imax * b.jmax * b.kmax;
-    const int cell = (blockIdx.x * 4 + w) * 64 + lane;
-    const bool ok = cell < ncell;
-    int L = 0;
-    EarsmT e;
-    bool in = false;
-    if (ok) {
-        const int i = cell % b.imax + 1, j = (cell / b.imax) % b.jmax + 1, k = cell / (b.imax * b.jmax) + 1;
-        L = cid(b, i, j, k);
-        earsm_terms(b, L, e);
-        float v[MNIN];
-        earsm_inputs(e, v);
-        in = true;
-        for (int q = 0; q < MNIN; q++) {
-            const float xn = (mlp_feature(v[q]) - nrm[MN_XM + q]) / nrm[MN_XS + q];
-            in = in && xn >= nrm[MN_LO + q] && xn <= nrm[MN_HI + q];
-            xs[w][lane][q] = xn;
-        }
-    } else {
-        for (int q = 0; q < MNIN; q++) xs[w][lane][q] = 0.f;
-    }
+    mlp_stage(p, wts);
     __syncthreads();
     MlpFrags f;
-    mlp_load_frags(p, lane, f, false);
+    mlp_load_frags(wts, lane, f, false);
+    for (long long base = 64ll * (blockIdx.x * 4 + w); base < ncell; base += 256ll * gridDim.x) {
+        const int cell = (int)base + lane;
+        const bool ok = cell < ncell;
+        int L = 0;
+        bool in = false;
+        if (ok) {
+            const int i = cell % b.imax + 1, j = (cell / b.imax) % b.jmax + 1, k = cell / (b.imax * b.jmax) + 1;
+            L = cid(b, i, j, k);
+            EarsmT e;
+            earsm_terms(b, L, e);
+            float v[MNIN];
+            earsm_inputs(e, v);
+            in = true;
+#pragma unroll
+            for (int q = 0; q < MNIN; q++) {
+                const float xn = (mlp_feature(v[q]) - nrm[MN_XM + q]) / nrm[MN_XS + q];
+                in = in && xn >= nrm[MN_LO + q] && xn <= nrm[MN_HI + q];
+                xs[w][lane][q] = xn;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < MNIN; q++) xs[w][lane][q] = 0.f;
+        }
+        wave_lds_sync();
 #pragma unroll 1
-    for (int cb = 0; cb < 4; cb++) {
-        float xn[4];
+        for (int cb = 0; cb < 4; cb++) {
+            float xn[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) xn[i] = 4 * g + i < MNIN ? xs[w][16 * cb + c][4 * g + i] : 0.f;
-        MlpFwd o;
-        mlp_forward16(f, lane, xn, o);
-        if (g == 0)
+            for (int i = 0; i < 4; i++) xn[i] = 4 * g + i < MNIN ? xs[w][16 * cb + c][4 * g + i] : 0.f;
+            MlpFwd o;
+            mlp_forward16(f, lane, xn, o);
+            if (g == 0)
 #pragma unroll
-            for (int i = 0; i < MNOUT; i++) ys[w][16 * cb + c][i] = mlp_output(o.y[i], nrm, i);
+                for (int i = 0; i < MNOUT; i++) ys[w][16 * cb + c][i] = o.y[i];
+        }
+        wave_lds_sync();
+        if (ok) {
+            // the tensor terms again (their ten fields are still in the L2): held through the
+            // network they took 50 registers a lane
+            EarsmT e;
+            earsm_terms(b, L, e);
+            double beta[4];
+            const double b6 = mlp_output(ys[w][lane][1], nrm, 1), b9 = mlp_output(ys[w][lane][2], nrm, 2);
+            if (in && b6 < 0. && b9 > 0.)
+                earsm_betas_n(e, -b6 / b9, beta);
+            else
+                earsm_betas(e, beta);
+            earsm_store(b, L, e, beta);
+        }
+        wave_lds_sync();
     }
-    __syncthreads();
-    if (!ok) return;
-    double beta[4];
-    const double b6 = ys[w][lane][1], b9 = ys[w][lane][2];
-    if (in && b6 < 0. && b9 > 0.)
-        earsm_betas_n(e, -b6 / b9, beta);
-    else
-        earsm_betas(e, beta);
-    earsm_store(b, L, e, beta);
 }
 
 static void mlp_free(MlpRec &r)
 {
     for (void *q : {(void *)r.p, (void *)r.m, (void *)r.v, (void *)r.nrm, (void *)r.nscr,
-                    (void *)r.part, (void *)r.idx, (void *)r.grad})
+                    (void *)r.part, (void *)r.loss, (void *)r.grad})
         if (q) (void)hipFree(q);
     r = MlpRec{};
 }
@@ -607,41 +690,42 @@ static int mlp_alloc(ff_ctx *c, MlpRec &r)
     return FF_OK;
 }
 
-static int mlp_workspace(ff_ctx *c, MlpRec &r, int waves, int nidx)
+// gradient partials of `parts` workgroups and device losses of `nloss` steps
+static int mlp_workspace(ff_ctx *c, MlpRec &r, int parts, int nloss)
 {
-    if (waves > r.part_waves) {
+    if (parts > r.parts) {
         if (r.part) (void)hipFree(r.part);
         r.part = nullptr;
-        r.part_waves = 0;
-        if (hipMalloc(&r.part, sizeof(float) * (size_t)MPP * waves) != hipSuccess)
+        r.parts = 0;
+        if (hipMalloc(&r.part, sizeof(float) * (size_t)MPP * parts) != hipSuccess)
             return fail(c, FF_E_NOMEM, "learned closure gradient partials%s");
-        r.part_waves = waves;
+        r.parts = parts;
     }
-    if (nidx > r.idx_cap) {
-        if (r.idx) (void)hipFree(r.idx);
-        r.idx = nullptr;
-        r.idx_cap = 0;
-        if (hipMalloc(&r.idx, sizeof(unsigned) * nidx) != hipSuccess)
-            return fail(c, FF_E_NOMEM, "learned closure minibatch%s");
-        r.idx_cap = nidx;
+    if (nloss > r.loss_cap) {
+        if (r.loss) (void)hipFree(r.loss);
+        r.loss = nullptr;
+        r.loss_cap = 0;
+        if (hipMalloc(&r.loss, sizeof(float) * nloss) != hipSuccess)
+            return fail(c, FF_E_NOMEM, "learned closure losses%s");
+        r.loss_cap = nloss;
     }
     return FF_OK;
 }
 
-// gradient over `nset` samples (all of them, or the minibatch in r.idx), reduced into r.grad;
-// with lr > 0 an Adam step as well
-static int mlp_grad_step(ff_ctx *c, MlpRec &r, const float *x, const float *y, const unsigned *idx,
-                         int nset, float lr)
+// gradient over `nset` samples (all of them, or a minibatch of bt.n), reduced into r.grad;
+// with lr > 0 an Adam step as well.  64 samples per workgroup (one pass of its waves) up to
+// 512 workgroups, which fill the chip twice; more samples loop.
+static int mlp_grad_step(ff_ctx *c, MlpRec &r, const float *x, const float *y, const MlpBatch &bt,
+                         int nset, float lr, float *loss)
 {
-    const int blocks = std::min(std::max((nset + 255) / 256, 1), 512);
-    const int waves = blocks * 4;
-    int rc = mlp_workspace(c, r, waves, 0);
+    const int blocks = std::min(std::max((nset + 63) / 64, 1), 512);
+    int rc = mlp_workspace(c, r, blocks, 0);
     if (rc) return rc;
     if ((rc = launch(c, "k_mlp_grad", k_mlp_grad, dim3(blocks), dim3(256), (const float *)r.p,
-                     (const float *)r.nrm, x, y, idx, nset, 1.0f / (float)nset, r.part))) return rc;
+                     (const float *)r.nrm, x, y, bt, nset, 1.0f / (float)nset, r.part))) return rc;
     if (lr > 0.f) r.step++;
-    return launch(c, "k_mlp_reduce", k_mlp_reduce, dim3((MPP + 255) / 256), dim3(256), r.p, r.m, r.v,
-                  (const float *)r.part, waves, lr, r.step, r.grad);
+    return launch(c, "k_mlp_reduce", k_mlp_reduce, dim3((MPP + RDC - 1) / RDC), dim3(RDC * RDS), r.p, r.m, r.v,
+                  (const float *)r.part, blocks, lr, r.step, r.grad, loss);
 }
 
 extern "C" {
@@ -714,7 +798,7 @@ int ff_mlp_infer(ff_ctx *c, const float *x, int n, float *y)
 {
     if (!c || !x || !y || n < 0) return FF_E_ARG;
     if (!c->mlp.ready) return fail(c, FF_E_STATE, "learned closure not set%s");
-    const int blocks = std::min(std::max((n + 63) / 64, 1), 4096);
+    const int blocks = std::min(std::max((n + 255) / 256, 1), MLP_GRID);
     int rc = launch(c, "k_mlp_infer", k_mlp_infer, dim3(blocks), dim3(256), (const float *)c->mlp.p,
                     (const float *)c->mlp.nrm, x, y, n);
     if (rc) return rc;
@@ -726,7 +810,7 @@ int ff_mlp_grad(ff_ctx *c, const float *x, const float *y, int n, float *grad)
 {
     if (!c || !x || !y || n < 1 || !grad) return FF_E_ARG;
     if (!c->mlp.ready) return fail(c, FF_E_STATE, "learned closure not set%s");
-    int rc = mlp_grad_step(c, c->mlp, x, y, nullptr, n, 0.f);
+    int rc = mlp_grad_step(c, c->mlp, x, y, MlpBatch{}, n, 0.f, nullptr);
     if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(grad, c->mlp.grad, sizeof(float) * MPP, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -738,15 +822,14 @@ int ff_mlp_train(ff_ctx *c, const float *x, const float *y, int n, int steps, in
 {
     if (!c || !x || !y || n < 1 || steps < 0 || batch < 16 || !(lr > 0.f)) return FF_E_ARG;
     if (!c->mlp.ready) return fail(c, FF_E_STATE, "learned closure not set%s");
-    int rc = mlp_workspace(c, c->mlp, 0, batch);
+    // the losses stay on the device until the last step (a copy per step waited for the host)
+    int rc = mlp_workspace(c, c->mlp, 0, loss ? steps : 0);
     if (rc) return rc;
-    for (int s = 0; s < steps; s++) {
-        if ((rc = launch(c, "k_mlp_batch", k_mlp_batch, dim3((batch + 255) / 256), dim3(256), c->mlp.idx,
-                         batch, n, seed, s))) return rc;
-        if ((rc = mlp_grad_step(c, c->mlp, x, y, c->mlp.idx, batch, lr))) return rc;
-        if (loss)
-            HIPCHK(c, hipMemcpyAsync(loss + s, c->mlp.grad + MNP, sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    }
+    for (int s = 0; s < steps; s++)
+        if ((rc = mlp_grad_step(c, c->mlp, x, y, MlpBatch{n, s, seed}, batch, lr, loss ? c->mlp.loss + s : nullptr)))
+            return rc;
+    if (loss && steps)
+        HIPCHK(c, hipMemcpyAsync(loss, c->mlp.loss, sizeof(float) * steps, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return FF_OK;
 }
@@ -757,6 +840,6 @@ int ff_mlp_train(ff_ctx *c, const float *x, const float *y, int n, int steps, in
 static int earsm_mlp_pass(ff_ctx *c, const Blk &b)
 {
     const int ncell = b.imax * b.jmax * b.kmax;
-    return launch(c, "k_earsm_mlp", k_earsm_mlp, dim3((ncell + 255) / 256), dim3(256), b,
+    return launch(c, "k_earsm_mlp", k_earsm_mlp, dim3(std::min((ncell + 255) / 256, MLP_GRID)), dim3(256), b,
                   (const float *)c->mlp.p, (const float *)c->mlp.nrm);
 }
