@@ -98,7 +98,7 @@ PHASE_OF = {"k_residual_kw": 0, "k_residual_kw_ns": 0, "k_residual_tile": 0,
             "k_residual_tile_ns": 0, "k_residual": 0,
             "k_pred_st": 1, "k_pred_tiles": 1, "k_pred_km": 1, "k_pred_plane": 1,
             "k_corr_st": 2, "k_corr_tiles": 2, "k_corr_km": 2, "k_corr_plane": 2}
-ALL_CELL_KERNELS = {"k_state", "k_save_old", "k_limits", "k_limits_mg", "k_forcing"}
+ALL_CELL_KERNELS = {"k_state", "k_save_old", "k_forcing", "k_fin"}
 # whole finest-level iteration, every field touched once per phase (residual; backward
 # sweep; forward sweep + update): laminar 88 doubles = 704 B, k-omega 110 doubles = 880 B
 ITER_BYTES_PER_CELL = {0: 704, 6: 880}
@@ -107,10 +107,10 @@ KERNELS = ("k_residual_kw", "k_residual_tile", "k_residual", "k_pred_tiles", "k_
            "k_sweep_prep", "k_pred_st", "k_corr_st", "k_wall", "k_wall_forces", "k_temder",
            "k_residual_kw_ns", "k_residual_tile_ns",
            "k_pred_km", "k_corr_km", "k_pred_plane", "k_corr_plane", "k_time3_copr", "k_state", "k_turb_lam",
-           "k_turb_sst", "k_grad_zero", "k_derfun", "k_extend", "k_crosko", "k_kw_round",
-           "k_max_final", "k_fun1_prod", "k_limits", "k_limits_mg", "k_fin", "k_zero", "k_fill_slots",
+           "k_turb_sst", "k_derfun", "k_crosko", "k_kw_round",
+           "k_fun1_prod", "k_fin", "k_zero", "k_fill_slots",
            "k_save_old", "k_divcp", "k_resl2_part", "k_resl2_final", "k_restrict",
-           "k_restrict_ghosts", "k_forcing", "k_prolong", "k_ddadi", "k_ddadi_end", "k_reflec")
+           "k_forcing", "k_prolong", "k_ddadi", "k_ddadi_end", "k_reflec")
 
 
 def make_workload(name="sst-mg", seed=0):

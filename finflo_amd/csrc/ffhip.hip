@@ -13,8 +13,8 @@
 //   k_pred_plane   PREDGS on one hyperplane I+J+K = m (imps4.f:345-598)
 //   k_corr_plane   DIAGGS + CORRGS on one hyperplane (imps4.f:604-664, 76-339)
 //   k_divcp        DRO/CP (imps3.f:483)
-//   k_fin          FIN (res3c.f:1122-1126)
-//   k_limits       UPLIM/LOLIM of T, U, V, W, PDTOP, LOLIMP (ns3c.f:1553-1596)
+//   k_fin          FIN (res3c.f:1122-1126), then UPLIM/LOLIM of T, U, V, W, PDTOP, LOLIMP
+//                  (ns3c.f:1553-1596)
 //
 // LU-SGS: the reference sweeps K-planes in order and, inside a plane, the diagonals
 // M = I+J (imps4.f:488-570, 221-308).  Every cell's update reads only the final increments
@@ -43,15 +43,29 @@ using namespace ff;
 // kernels
 // ------------------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(256) k_state(Prm p, Blk b)
+// SAVE: at the start of a cycle, the OLD copies of the solved variables as well (k_save_old,
+// with the cycle count of a block with INL/OUT patches); one pass reads the variables once
+// (192x96x96 laminar: 36 + 47 us as two passes, 67 as one).
+template <bool SAVE>
+__global__ void __launch_bounds__(256) k_state(Prm p, Blk b, int *icyc)
 {
     int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (SAVE && icyc && n == 0) *icyc = *icyc + 1;
     if (n >= b.ntot) return;
     const double gm1 = p.gamma - 1.;
     const double cp2 = p.gamma / gm1 * p.rgas;
     const double cmin = 1.;
     double pd = FLD(b, FF_PDIFF)[n], t = FLD(b, FF_TEMP)[n];
     double u = FLD(b, FF_U)[n], v = FLD(b, FF_V)[n], w = FLD(b, FF_W)[n];
+    if (SAVE) {
+        FLD(b, FF_TOLD)[n] = t;
+        FLD(b, FF_UOLD)[n] = u;
+        FLD(b, FF_VOLD)[n] = v;
+        FLD(b, FF_WOLD)[n] = w;
+        FLD(b, FF_POLD)[n] = pd;
+        FLD(b, FF_RKOLD)[n] = FLD(b, FF_RK)[n];
+        FLD(b, FF_EPSOLD)[n] = FLD(b, FF_REPS)[n];
+    }
     double P = pd + p.frspre;                                   // PDTOP state.f:1707
     double trgs = t * p.rgas;                                   // PERFGA state.f:212-229
     double drdp = 1. / trgs;
@@ -108,8 +122,9 @@ __global__ void __launch_bounds__(256) k_turb_lam(Blk b)
 __device__ __forceinline__ double pow4(double x) { return x * x * x * x; }   // ((x*x)*x)*x
 
 // DERFUN (turb3.f:2539-2665, IDERI = 1) at cell L: velocity gradients by distance-weighted
-// Green-Gauss, stored as vorticity, strain rate, |Omega| (OHMI) and strain magnitude
-__device__ __forceinline__ double derfun_cell(const Blk &b, int L)
+// Green-Gauss, stored as vorticity, strain rate, |Omega| (OHMI) and, strn, strain magnitude at
+// cell to
+__device__ __forceinline__ double derfun_cell(const Blk &b, int L, int to, bool strn = true)
 {
     const int IS = b.is, IL = b.il;
     const double *u = FLD(b, FF_U), *v = FLD(b, FF_V), *w = FLD(b, FF_W);
@@ -154,16 +169,16 @@ __device__ __forceinline__ double derfun_cell(const Blk &b, int L)
     const double dvdx = g[0][1], dvdy = g[1][1], dvdz = g[2][1];
     const double dwdx = g[0][2], dwdy = g[1][2], dwdz = g[2][2];
     double w12 = .5 * (dudy - dvdx), w13 = .5 * (dudz - dwdx), w23 = .5 * (dvdz - dwdy);
-    FLD(b, FF_W12)[L] = w12; FLD(b, FF_W13)[L] = w13; FLD(b, FF_W23)[L] = w23;
-    FLD(b, FF_OHMI)[L] = 2. * sqrt(w12 * w12 + w13 * w13 + w23 * w23);
+    FLD(b, FF_W12)[to] = w12; FLD(b, FF_W13)[to] = w13; FLD(b, FF_W23)[to] = w23;
+    FLD(b, FF_OHMI)[to] = 2. * sqrt(w12 * w12 + w13 * w13 + w23 * w23);
     double s11 = .5 * (dudx + dudx), s22 = .5 * (dvdy + dvdy), s33 = .5 * (dwdz + dwdz);
     double s12 = .5 * (dudy + dvdx), s13 = .5 * (dudz + dwdx), s23 = .5 * (dvdz + dwdy);
     double st = s11 * s11 + s12 * s12 + s13 * s13 + s12 * s12 + s22 * s22 + s23 * s23
               + s13 * s13 + s23 * s23 + s33 * s33;
     const double strain = sqrt(2. * st);
-    FLD(b, FF_STRAIN)[L] = strain;
-    FLD(b, FF_S11)[L] = s11; FLD(b, FF_S12)[L] = s12; FLD(b, FF_S13)[L] = s13;
-    FLD(b, FF_S22)[L] = s22; FLD(b, FF_S23)[L] = s23; FLD(b, FF_S33)[L] = s33;
+    if (strn) FLD(b, FF_STRAIN)[to] = strain;
+    FLD(b, FF_S11)[to] = s11; FLD(b, FF_S12)[to] = s12; FLD(b, FF_S13)[to] = s13;
+    FLD(b, FF_S22)[to] = s22; FLD(b, FF_S23)[to] = s23; FLD(b, FF_S33)[to] = s33;
     return strain;
 }
 
@@ -330,7 +345,7 @@ __global__ void __launch_bounds__(256) k_turb_sst(Prm p, Blk b)
     int j = blockIdx.y, k = blockIdx.z;
     if (i >= ni) return;
     const int L = cid(b, i, j, k);
-    const double strain = derfun_cell(b, L);
+    const double strain = derfun_cell(b, L, L);
     // TTIMES
     const double ro = FLD(b, FF_RO)[L], vis = FLD(b, FF_VIS)[L];
     const double rk = FLD(b, FF_RK)[L], rom = FLD(b, FF_REPS)[L];
@@ -372,25 +387,35 @@ __global__ void __launch_bounds__(256) k_turb_sst(Prm p, Blk b)
     FLD(b, FF_EPS2)[L] = 1.0 + rmutpv;
 }
 
-// RESIKE with M2 >= 2 (res3c.f:3749-3769): OHMI, W12 and SIJ zeroed on every cell, then
-// DERFUN on level 1 with the first ghost layer (g0 = 1) or on a coarse level's interior
-// (g0 = 0).  Thread per cell of the range.
-constexpr int NGRAD = 10;
-__global__ void __launch_bounds__(256) k_grad_zero(Blk b)
-{
-    int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= b.ntot) return;
-    FLD(b, FF_OHMI)[n] = 0.;
-#pragma unroll
-    for (int q = 0; q < 9; q++) FLD(b, FF_W12 + q)[n] = 0.;
-}
-
 __global__ void __launch_bounds__(256) k_derfun(Blk b, int g0)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x + 1 - g0;
     int j = blockIdx.y + 1 - g0, k = blockIdx.z + 1 - g0;
     if (i > b.imax + g0) return;
-    derfun_cell(b, cid(b, i, j, k));
+    derfun_cell(b, cid(b, i, j, k), cid(b, i, j, k));
+}
+
+// RESIKE with M2 >= 2 (res3c.f:3749-3769) on every cell, thread per cell with I fastest: DERFUN
+// on level 1 with the first ghost layer (g0 = 1), or on a coarse level's interior with EXTEND
+// (turb3.f:3342-3450: the interior value next to each face copied into the first ghost layer,
+// no edges or corners); OHMI, W12 and SIJ are zero everywhere else.  A ghost cell of EXTEND
+// forms its interior neighbour's gradients again, the same operations on the same operands:
+// one pass for the three of ZEROZZ, DERFUN and EXTEND.
+__global__ void __launch_bounds__(256) k_gradients(Blk b, int g0)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x - 1, j = (int)blockIdx.y - 1, k = (int)blockIdx.z - 1;
+    if (i > b.imax + 2) return;
+    const int n = cid(b, i, j, k);
+    auto out = [](int x, int m) { return x < 1 ? 1 - x : x > m ? x - m : 0; };
+    const int oi = out(i, b.imax), oj = out(j, b.jmax), ok = out(k, b.kmax);
+    if (g0 ? oi <= 1 && oj <= 1 && ok <= 1 : oi + oj + ok <= 1) {
+        const int src = g0 ? n : cid(b, min(max(i, 1), b.imax), min(max(j, 1), b.jmax), min(max(k, 1), b.kmax));
+        derfun_cell(b, src, n, g0 || oi + oj + ok == 0);
+        return;
+    }
+    FLD(b, FF_OHMI)[n] = 0.;
+#pragma unroll
+    for (int q = 0; q < 9; q++) FLD(b, FF_W12 + q)[n] = 0.;
 }
 
 // TEMDER turb3.f:3456-3559, IDERI = 1, of the cell scalar q (gq picks it) at cell L: the
@@ -452,30 +477,6 @@ __global__ void __launch_bounds__(256) k_temder(Blk b, int gk)
     }
 }
 
-// EXTEND (turb3.f:3342-3450) of OHMI, W12 and SIJ on a coarse level: the interior value
-// next to each face copied into the first ghost layer (no edges or corners)
-__global__ void __launch_bounds__(256) k_extend(Blk b)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    int j = blockIdx.y + 1, k = blockIdx.z + 1;
-    if (i > b.imax) return;
-    const int n = cid(b, i, j, k);
-    const int IS = b.is, IL = b.il;
-    int t[6], nt = 0;
-    if (k == 1) t[nt++] = n - IL;
-    if (k == b.kmax) t[nt++] = n + IL;
-    if (j == 1) t[nt++] = n - IS;
-    if (j == b.jmax) t[nt++] = n + IS;
-    if (i == 1) t[nt++] = n - 1;
-    if (i == b.imax) t[nt++] = n + 1;
-    if (nt == 0) return;
-    for (int q = 0; q < NGRAD; q++) {
-        double *x = FLD(b, q == 0 ? FF_OHMI : FF_W12 + q - 1);
-        double v = x[n];
-        for (int r = 0; r < nt; r++) x[t[r]] = v;
-    }
-}
-
 // ------------------------------------------------------------------------------------
 // multigrid transfers (multi.f)
 // ------------------------------------------------------------------------------------
@@ -494,20 +495,25 @@ __device__ __forceinline__ double restrict8(const Blk &f, const double *vol, con
             vol[ipjkp] * x[ipjkp] + vol[ijpkp] * x[ijpkp]) * pvol;
 }
 
-// TRANSF (+ TRANKE, KW) loop 1000 and the OLD copies (multi.f:194-278, 453-510): coarse cell
-// per thread over the interior and the first ghost layer.  A planar fine level (KMAX = 1)
-// maps coarse K to fine K (KIND = 1, multi.f:185-196).
+// TRANSF (+ TRANKE, KW): loop 1000 with the OLD copies (multi.f:194-278, 453-510) and the ghost
+// treatment of loops 2100-2600 (multi.f:283-425), coarse cell per thread over the whole slab.
+// The loops take the interior and the first ghost layer from the fine cells, zero the
+// residual transfers on both ghost layers and copy the variables from the first to the
+// second, I, J and K in turn: a cell of the second layer ends with the value of the cell its
+// indices clamp to in 0..N+1, which it forms here again (one launch for four).  A planar fine
+// level (KMAX = 1) maps coarse K to fine K (KIND = 1, multi.f:185-196).
 template <bool KW>
 __global__ void __launch_bounds__(256) k_restrict(Blk f, Blk c)
 {
-    int I = blockIdx.x * blockDim.x + threadIdx.x;
-    int J = blockIdx.y, K = blockIdx.z;
-    if (I > c.imax + 1) return;
-    const int n = cid(c, I, J, K);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x - 1, j = (int)blockIdx.y - 1, k = (int)blockIdx.z - 1;
+    if (i > c.imax + 2) return;
+    const int n = cid(c, i, j, k);
+    const int I = min(max(i, 0), c.imax + 1), J = min(max(j, 0), c.jmax + 1), K = min(max(k, 0), c.kmax + 1);
+    const bool in = i >= 1 && i <= c.imax && j >= 1 && j <= c.jmax && k >= 1 && k <= c.kmax;
     const bool planar = f.kmax == 1;
     const int ijk = cid(f, 2 * I - 1, 2 * J - 1, planar ? K : 2 * K - 1), kp = planar ? 0 : f.il;
     const double *vol = FLD(f, FF_VOL);
-    const double pvol = 1. / FLD(c, FF_VOL)[n];
+    const double pvol = 1. / FLD(c, FF_VOL)[cid(c, I, J, K)];
     const int st[7] = {FF_TEMP, FF_U, FF_V, FF_W, FF_PDIFF, FF_EPS2, FF_VIST};
     double x[7];
 #pragma unroll
@@ -516,17 +522,17 @@ __global__ void __launch_bounds__(256) k_restrict(Blk f, Blk c)
         FLD(c, st[q])[n] = x[q];
     }
 #pragma unroll
-    for (int q = 0; q < 5; q++) FLD(c, FF_ROP2H + q)[n] = restrict8(f, vol, FLD(f, FF_DRO + q), ijk, kp, pvol);
+    for (int q = 0; q < 5; q++) FLD(c, FF_ROP2H + q)[n] = in ? restrict8(f, vol, FLD(f, FF_DRO + q), ijk, kp, pvol) : 0.;
     double rk = 0., re = 0.;
     if (KW) {
         rk = restrict8(f, vol, FLD(f, FF_RK), ijk, kp, pvol);
         re = restrict8(f, vol, FLD(f, FF_REPS), ijk, kp, pvol);
         FLD(c, FF_RK)[n] = rk;
         FLD(c, FF_REPS)[n] = re;
-        FLD(c, FF_RKP2H)[n] = restrict8(f, vol, FLD(f, FF_DRK), ijk, kp, pvol);
-        FLD(c, FF_EPSP2H)[n] = restrict8(f, vol, FLD(f, FF_DEPS), ijk, kp, pvol);
+        FLD(c, FF_RKP2H)[n] = in ? restrict8(f, vol, FLD(f, FF_DRK), ijk, kp, pvol) : 0.;
+        FLD(c, FF_EPSP2H)[n] = in ? restrict8(f, vol, FLD(f, FF_DEPS), ijk, kp, pvol) : 0.;
     }
-    if (I >= 1 && I <= c.imax && J >= 1 && J <= c.jmax && K >= 1 && K <= c.kmax) {
+    if (in) {
         FLD(c, FF_TOLD)[n] = x[0];
         FLD(c, FF_UOLD)[n] = x[1];
         FLD(c, FF_VOLD)[n] = x[2];
@@ -539,114 +545,79 @@ __global__ void __launch_bounds__(256) k_restrict(Blk f, Blk c)
     }
 }
 
-// The ghost treatment of TRANSF/TRANKE (loops 2100-2600, multi.f:283-425) for one pair of
-// opposite faces: face 0 = I, 1 = J, 2 = K.  Residual transfers are zeroed on both ghost
-// layers and the variables copied from the first to the second; the launches for I, J and
-// K run in that order, as the reference's loops do.
-template <bool KW>
-__global__ void __launch_bounds__(256) k_restrict_ghosts(Blk c, int face)
-{
-    const int na = (face == 0 ? c.jmax : c.imax) + 4;          // index a runs over -1..N+2
-    int a = blockIdx.x * blockDim.x + threadIdx.x - 1;
-    int bb = blockIdx.y - 1;                                   // the other index
-    if (a > na - 2) return;
-    int lo, hi, st;
-    if (face == 0) {        // (J = a, K = bb)
-        lo = cid(c, 0, a, bb); hi = cid(c, c.imax + 1, a, bb); st = 1;
-    } else if (face == 1) { // (I = a, K = bb)
-        lo = cid(c, a, 0, bb); hi = cid(c, a, c.jmax + 1, bb); st = c.is;
-    } else {                // (I = a, J = bb)
-        lo = cid(c, a, bb, 0); hi = cid(c, a, bb, c.kmax + 1); st = c.il;
-    }
-    const int nz = KW ? 7 : 5;
-    for (int q = 0; q < nz; q++) {
-        double *x = FLD(c, FF_ROP2H + q);
-        x[lo] = 0.; x[lo - st] = 0.; x[hi] = 0.; x[hi + st] = 0.;
-    }
-    const int cp[9] = {FF_TEMP, FF_U, FF_V, FF_W, FF_PDIFF, FF_EPS2, FF_VIST, FF_RK, FF_REPS};
-    const int ncp = KW ? 9 : 7;
-    for (int q = 0; q < ncp; q++) {
-        double *x = FLD(c, cp[q]);
-        x[lo - st] = x[lo];
-        x[hi + st] = x[hi];
-    }
-}
-
 // FORCFU (phase 0, P = P - D, multi.f:1630-1648) or ADDRES (phase 1, D = P + D,
-// multi.f:1707-1725) on every cell
+// multi.f:1707-1725) on every cell; phase 2: one after the other
 __global__ void __launch_bounds__(256) k_forcing(Blk b, int nq, int phase)
 {
     int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= b.ntot) return;
     for (int q = 0; q < nq; q++) {
         double *P = FLD(b, FF_ROP2H + q), *D = FLD(b, FF_DRO + q);
-        if (phase == 0) P[n] = P[n] - D[n];
-        else D[n] = P[n] + D[n];
+        double x = P[n], d = D[n];
+        if (phase != 1) {
+            x = x - d;
+            P[n] = x;
+        }
+        if (phase != 0) D[n] = x + d;
     }
 }
 
-// INTERP (multi.f:1790-1819) and, KW, INTERT/INTERO (multi.f:2007-2077): fine interior cell
-// per thread, the correction of coarse cell ((I+1)/2, (J+1)/2, (K+1)/2)
+// INTERP (multi.f:1790-1819) and, KW, INTERT/INTERO (multi.f:2007-2077): a fine interior cell
+// takes the correction of coarse cell ((I+1)/2, (J+1)/2, (K+1)/2); then, on every cell, the
+// limiters CYCLES applies after the prolongation (ns3c.f:2073-2118: for two-equation models
+// the TEMP limits and LOLIM of RK and REPS, then LOLIMP with the level's last pressure).
+// Thread per cell of the fine slab.
 template <bool KW>
 __global__ void __launch_bounds__(256) k_prolong(Prm p, Blk c, Blk f)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    int j = blockIdx.y + 1, k = blockIdx.z + 1;
-    if (i > f.imax) return;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x - 1, j = (int)blockIdx.y - 1, k = (int)blockIdx.z - 1;
+    if (i > f.imax + 2) return;
     const int ijk = cid(f, i, j, k);
-    const int n = cid(c, (i + 1) / 2, (j + 1) / 2, (k + 1) / 2);
-    double dtok = FLD(c, FF_TEMP)[n] - FLD(c, FF_TOLD)[n];
-    double duk = FLD(c, FF_U)[n] - FLD(c, FF_UOLD)[n];
-    double dvk = FLD(c, FF_V)[n] - FLD(c, FF_VOLD)[n];
-    double dwk = FLD(c, FF_W)[n] - FLD(c, FF_WOLD)[n];
-    double dpk = FLD(c, FF_PDIFF)[n] - FLD(c, FF_POLD)[n];
-    FLD(f, FF_TEMP)[ijk] = FLD(f, FF_TEMP)[ijk] + dtok;
-    FLD(f, FF_U)[ijk] = FLD(f, FF_U)[ijk] + duk;
-    FLD(f, FF_V)[ijk] = FLD(f, FF_V)[ijk] + dvk;
-    FLD(f, FF_W)[ijk] = FLD(f, FF_W)[ijk] + dwk;
-    FLD(f, FF_P)[ijk] = FLD(f, FF_P)[ijk] + dpk;
-    FLD(f, FF_PDIFF)[ijk] = FLD(f, FF_PDIFF)[ijk] + dpk;
+    const bool up = j >= 1 && j <= f.jmax && k >= 1 && k <= f.kmax, in = up && i >= 1 && i <= f.imax;
+    double P = FLD(f, FF_P)[ijk], pd = FLD(f, FF_PDIFF)[ijk], t = 0., tk[2] = {0., 0.};
+    if (KW || in) t = FLD(f, FF_TEMP)[ijk];
     if (KW) {
-        const double eps = 1.E-7;
+        tk[0] = FLD(f, FF_RK)[ijk];
+        tk[1] = FLD(f, FF_REPS)[ijk];
+    }
+    if (in) {
+        const int n = cid(c, (i + 1) / 2, (j + 1) / 2, (k + 1) / 2);
+        double dtok = FLD(c, FF_TEMP)[n] - FLD(c, FF_TOLD)[n];
+        double duk = FLD(c, FF_U)[n] - FLD(c, FF_UOLD)[n];
+        double dvk = FLD(c, FF_V)[n] - FLD(c, FF_VOLD)[n];
+        double dwk = FLD(c, FF_W)[n] - FLD(c, FF_WOLD)[n];
+        double dpk = FLD(c, FF_PDIFF)[n] - FLD(c, FF_POLD)[n];
+        t = t + dtok;
+        FLD(f, FF_U)[ijk] = FLD(f, FF_U)[ijk] + duk;
+        FLD(f, FF_V)[ijk] = FLD(f, FF_V)[ijk] + dvk;
+        FLD(f, FF_W)[ijk] = FLD(f, FF_W)[ijk] + dwk;
+        P = P + dpk;
+        pd = pd + dpk;
+        if (KW) {
+            const double eps = 1.E-7;
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const double cc1 = q == 0 ? p.cmgk : p.cmgeps, cc2 = cc1 + eps;
-            double *ro = FLD(f, q == 0 ? FF_RK : FF_REPS);
-            double drok = FLD(c, q == 0 ? FF_RK : FF_REPS)[n] - FLD(c, q == 0 ? FF_RKOLD : FF_EPSOLD)[n];
-            double alpo = fabs(drok);
-            double r = ro[ijk];
-            ro[ijk] = r + cc1 * r * drok / (cc2 * r + alpo);
+            for (int q = 0; q < 2; q++) {
+                const double cc1 = q == 0 ? p.cmgk : p.cmgeps, cc2 = cc1 + eps;
+                double drok = FLD(c, q == 0 ? FF_RK : FF_REPS)[n] - FLD(c, q == 0 ? FF_RKOLD : FF_EPSOLD)[n];
+                double alpo = fabs(drok);
+                double r = tk[q];
+                tk[q] = r + cc1 * r * drok / (cc2 * r + alpo);
+            }
+        } else {
+            FLD(f, FF_TEMP)[ijk] = t;
         }
     }
-}
-
-// The limiters CYCLES applies on a level other than the finest after FIN (ns3c.f:1936-1985:
-// UPLIM/LOLIM of TEMP, LOLIMP with the level's last pressure) or on a level after the
-// prolongation into it (ns3c.f:2073-2118: for two-equation models the TEMP limits and LOLIM of
-// RK and REPS, then LOLIMP).  Every cell.
-__global__ void __launch_bounds__(256) k_limits_mg(Prm p, Blk b, int temp_limits, int kw_limits)
-{
-    int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= b.ntot) return;
-    if (temp_limits) {
-        int kk = n / b.il;
-        int jj = (n / b.is) % b.js;
-        bool up = kk >= 2 && kk < 2 + b.kmax && jj >= 2 && jj < 2 + b.jmax;
-        double t = FLD(b, FF_TEMP)[n];
+    if (KW) {
         if (up) t = t < p.tuplim ? t : p.tuplim;
         t = t > p.tlolim ? t : p.tlolim;
-        FLD(b, FF_TEMP)[n] = t;
+        FLD(f, FF_TEMP)[ijk] = t;
+        FLD(f, FF_RK)[ijk] = tk[0] > p.rklim ? tk[0] : p.rklim;
+        FLD(f, FF_REPS)[ijk] = tk[1] > p.epslim ? tk[1] : p.epslim;
     }
-    if (kw_limits) {
-        double rk = FLD(b, FF_RK)[n], re = FLD(b, FF_REPS)[n];
-        FLD(b, FF_RK)[n] = rk > p.rklim ? rk : p.rklim;
-        FLD(b, FF_REPS)[n] = re > p.epslim ? re : p.epslim;
-    }
-    double P = FLD(b, FF_P)[n];
     double y = P - 0.01 * p.frspre;
     double prelim = 0. < y ? 0. : y;
-    FLD(b, FF_P)[n] = P - prelim;
-    FLD(b, FF_PDIFF)[n] = FLD(b, FF_PDIFF)[n] - prelim;
+    FLD(f, FF_P)[ijk] = P - prelim;
+    FLD(f, FF_PDIFF)[ijk] = pd - prelim;
 }
 
 // k = RK/RO and omega = REPS/RO as CROSKO forms them in place (turb3.f:7817-7821)
@@ -657,9 +628,11 @@ __device__ __forceinline__ double per_ro(const double *x, const double *ro, int 
 }
 
 // CROSKO turb3.f:7824-7892 on the interior: SEPS = 2*SIGOM2*RO*grad(k).grad(omega)/omega,
-// with k and omega formed from the unrounded RK, REPS of each stencil cell
-__global__ void __launch_bounds__(256) k_crosko(Prm p, Blk b)
+// with k and omega formed from the unrounded RK, REPS of each stencil cell.  Clears the
+// maximum k_kw_round takes next.
+__global__ void __launch_bounds__(256) k_crosko(Prm p, Blk b, double *cdmax)
 {
+    if (blockIdx.x + blockIdx.y + blockIdx.z + threadIdx.x == 0) *cdmax = 0.;
     int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     int j = blockIdx.y + 1, k = blockIdx.z + 1;
     if (i > b.imax) return;
@@ -690,9 +663,11 @@ __global__ void __launch_bounds__(256) k_crosko(Prm p, Blk b)
 }
 
 // The rounding CROSKO leaves on RK and REPS of every cell: (X*(1/RO))*RO (turb3.f:7895-7898).
-// Also zeroes FUN1 and SRK (RESIKE res3c.f:3673, 3730) and forms per-workgroup maxima of
-// SEPS over the linear index range FUN1KO scans (turb3.f:7423-7428).
-__global__ void __launch_bounds__(256) k_kw_round(Blk b, double *part)
+// Also zeroes FUN1, SRK and the residuals DRO.. (ZEROZZ, RESIKE res3c.f:3668-3674, 3730) and
+// takes the maximum of SEPS, at least zero, over the linear index range FUN1KO scans
+// (turb3.f:7423-7428): an integer maximum, since the bits of non-negative doubles order as
+// their values (and a maximum is exact in any order).
+__global__ void __launch_bounds__(256) k_kw_round(Blk b, double *cdmax)
 {
     __shared__ double sh[256];
     int n = blockIdx.x * blockDim.x + threadIdx.x;
@@ -703,7 +678,9 @@ __global__ void __launch_bounds__(256) k_kw_round(Blk b, double *part)
         FLD(b, FF_REPS)[n] = per_ro(FLD(b, FF_REPS), FLD(b, FF_RO), n) * ro;
         FLD(b, FF_FUN1)[n] = 0.;
         FLD(b, FF_SRK)[n] = 0.;
-        if (n >= cid(b, 1, 1, 1) && n <= cid(b, b.imax, b.jmax, b.kmax)) m = FLD(b, FF_SEPS)[n];
+#pragma unroll
+        for (int q = 0; q < 7; q++) FLD(b, FF_DRO + q)[n] = 0.;
+        if (n >= cid(b, 1, 1, 1) && n <= cid(b, b.imax, b.jmax, b.kmax)) m = dmax(FLD(b, FF_SEPS)[n], m);
     }
     sh[threadIdx.x] = m;
     __syncthreads();
@@ -711,22 +688,7 @@ __global__ void __launch_bounds__(256) k_kw_round(Blk b, double *part)
         if (threadIdx.x < h) sh[threadIdx.x] = dmax(sh[threadIdx.x + h], sh[threadIdx.x]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-// Maximum of the partial maxima (max is exact, so the order does not matter)
-__global__ void __launch_bounds__(256) k_max_final(const double *part, int nparts, double *out)
-{
-    __shared__ double sh[256];
-    double m = 0.0;
-    for (int t = threadIdx.x; t < nparts; t += blockDim.x) m = dmax(part[t], m);
-    sh[threadIdx.x] = m;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if (threadIdx.x < h) sh[threadIdx.x] = dmax(sh[threadIdx.x + h], sh[threadIdx.x]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = sh[0];
+    if (threadIdx.x == 0 && sh[0] > 0.) atomicMax((unsigned long long *)cdmax, (unsigned long long)__double_as_longlong(sh[0]));
 }
 
 // FUN1KO (turb3.f:7430-7446) and PRODKE (turb3.f:4720-4787, with MAKE_EPS turb3.f:7913)
@@ -3835,12 +3797,10 @@ __global__ void __launch_bounds__(256) k_divcp(Blk b)
     FLD(b, FF_DRO)[n] = FLD(b, FF_DRO)[n] / FLD(b, FF_CP)[n];
 }
 
-// Start-of-cycle copies (TOLD ...) on every cell; a cycle of a block with INL/OUT patches
-// also counts its ICYCLE (icyc, null otherwise)
-__global__ void __launch_bounds__(256) k_save_old(Blk b, int *icyc)
+// Start-of-cycle copies (TOLD ...) on every cell (a cycle takes them with its state)
+__global__ void __launch_bounds__(256) k_save_old(Blk b)
 {
     int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (icyc && n == 0) *icyc = *icyc + 1;
     if (n >= b.ntot) return;
     FLD(b, FF_TOLD)[n] = FLD(b, FF_TEMP)[n];
     FLD(b, FF_UOLD)[n] = FLD(b, FF_U)[n];
@@ -3851,78 +3811,63 @@ __global__ void __launch_bounds__(256) k_save_old(Blk b, int *icyc)
     FLD(b, FF_EPSOLD)[n] = FLD(b, FF_REPS)[n];
 }
 
-// FIN (res3c.f:1122-1126) on interior cells
-__global__ void __launch_bounds__(256) k_fin(Blk b)
+// FIN (res3c.f:1122-1126; the relaxed update of rho*k and rho*omega res3c.f:1182-1198) on the
+// interior cells, then the limiters on every cell: on level 1 those of CYCLES (ns3c.f:1553-
+// 1596: UPLIM acts on interior K-planes and J-rows, all I, res3c.f:3401-3417, LOLIM / PDTOP /
+// LOLIMP on all cells), on a coarse level those of ns3c.f:1936-1985 (UPLIM/LOLIM of TEMP,
+// LOLIM of RK and REPS, LOLIMP with the level's last pressure).  One pass reads and writes the
+// solved variables once (192x96x96 laminar: 36 + 29 us as two passes, 41 as one).
+template <bool KW, bool COARSE>
+__global__ void __launch_bounds__(256) k_fin(Prm p, Blk b)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    int j = blockIdx.y + 1;
-    int k = blockIdx.z + 1;
-    if (i > b.imax) return;
-    int n = cid(b, i, j, k);
-    FLD(b, FF_TEMP)[n] = FLD(b, FF_TOLD)[n] + FLD(b, FF_DRO)[n];
-    FLD(b, FF_U)[n] = FLD(b, FF_UOLD)[n] + FLD(b, FF_DM)[n];
-    FLD(b, FF_V)[n] = FLD(b, FF_VOLD)[n] + FLD(b, FF_DN)[n];
-    FLD(b, FF_W)[n] = FLD(b, FF_WOLD)[n] + FLD(b, FF_DW)[n];
-    FLD(b, FF_PDIFF)[n] = FLD(b, FF_POLD)[n] + FLD(b, FF_DE)[n];
-}
-
-// FIN for two-equation models (res3c.f:1182-1198): the mean flow as above plus the relaxed
-// update of rho*k and rho*omega
-__global__ void __launch_bounds__(256) k_fin_kw(Blk b)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    int j = blockIdx.y + 1;
-    int k = blockIdx.z + 1;
-    if (i > b.imax) return;
-    int n = cid(b, i, j, k);
-    FLD(b, FF_TEMP)[n] = FLD(b, FF_TOLD)[n] + FLD(b, FF_DRO)[n];
-    FLD(b, FF_U)[n] = FLD(b, FF_UOLD)[n] + FLD(b, FF_DM)[n];
-    FLD(b, FF_V)[n] = FLD(b, FF_VOLD)[n] + FLD(b, FF_DN)[n];
-    FLD(b, FF_W)[n] = FLD(b, FF_WOLD)[n] + FLD(b, FF_DW)[n];
-    FLD(b, FF_PDIFF)[n] = FLD(b, FF_POLD)[n] + FLD(b, FF_DE)[n];
-    double rko = FLD(b, FF_RKOLD)[n], epo = FLD(b, FF_EPSOLD)[n];
-    double drk = FLD(b, FF_DRK)[n], dep = FLD(b, FF_DEPS)[n];
-    double rkoldn = .45 * rko;
-    double epoldn = .90 * epo;
-    double absdrk = fabs(drk);
-    double absdep = fabs(dep);
-    FLD(b, FF_RK)[n] = rko + drk / (1. + absdrk / rkoldn);
-    FLD(b, FF_REPS)[n] = epo + dep / (1. + absdep / epoldn);
-}
-
-// Limiters of CYCLES (ns3c.f:1553-1596) on every cell: UPLIM acts on interior K-planes and
-// J-rows (all I, res3c.f:3401-3417), LOLIM / PDTOP / LOLIMP on all cells.
-__global__ void __launch_bounds__(256) k_limits(Prm p, Blk b)
-{
-    int n = blockIdx.x * blockDim.x + threadIdx.x;
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= b.ntot) return;
-    int kk = n / b.il;
-    int jj = (n / b.is) % b.js;
-    bool up = kk >= 2 && kk < 2 + b.kmax && jj >= 2 && jj < 2 + b.jmax;
-    double *x;
-    x = FLD(b, FF_TEMP);
-    double t = x[n];
+    const int kk = n / b.il, jj = (n / b.is) % b.js, ii = n % b.is;
+    const bool up = kk >= 2 && kk < 2 + b.kmax && jj >= 2 && jj < 2 + b.jmax;
+    const bool in = up && ii >= 2 && ii < 2 + b.imax;
+    double t, s[3], pd, rk = 0., re = 0.;
+    if (in) {
+        t = FLD(b, FF_TOLD)[n] + FLD(b, FF_DRO)[n];
+#pragma unroll
+        for (int q = 0; q < 3; q++) s[q] = FLD(b, FF_UOLD + q)[n] + FLD(b, FF_DM + q)[n];
+        pd = FLD(b, FF_POLD)[n] + FLD(b, FF_DE)[n];
+        if (KW) {
+            double rko = FLD(b, FF_RKOLD)[n], epo = FLD(b, FF_EPSOLD)[n];
+            double drk = FLD(b, FF_DRK)[n], dep = FLD(b, FF_DEPS)[n];
+            double rkoldn = .45 * rko;
+            double epoldn = .90 * epo;
+            rk = rko + drk / (1. + fabs(drk) / rkoldn);
+            re = epo + dep / (1. + fabs(dep) / epoldn);
+        }
+    } else {
+        t = FLD(b, FF_TEMP)[n];
+#pragma unroll
+        for (int q = 0; q < 3; q++) s[q] = FLD(b, FF_U + q)[n];
+        pd = FLD(b, FF_PDIFF)[n];
+        if (KW) {
+            rk = FLD(b, FF_RK)[n];
+            re = FLD(b, FF_REPS)[n];
+        }
+    }
     if (up) t = t < p.tuplim ? t : p.tuplim;
     t = t > p.tlolim ? t : p.tlolim;
-    x[n] = t;
+    FLD(b, FF_TEMP)[n] = t;
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        x = FLD(b, FF_U + q);
-        double s = x[n];
-        if (up) s = s < 5000. ? s : 5000.;
-        s = s > -5000. ? s : -5000.;
-        x[n] = s;
+        if (!COARSE) {
+            if (up) s[q] = s[q] < 5000. ? s[q] : 5000.;
+            s[q] = s[q] > -5000. ? s[q] : -5000.;
+        }
+        if (!COARSE || in) FLD(b, FF_U + q)[n] = s[q];
     }
-    if (p.iturb == 6) {
+    if (KW) {
         // LOLIM of RK and REPS (FIN res3c.f:1202-1205; CYCLES ns3c.f:1575-1576)
-        double rk = FLD(b, FF_RK)[n], re = FLD(b, FF_REPS)[n];
         FLD(b, FF_RK)[n] = rk > p.rklim ? rk : p.rklim;
         FLD(b, FF_REPS)[n] = re > p.epslim ? re : p.epslim;
     }
-    double pd = FLD(b, FF_PDIFF)[n];
-    double P = pd + p.frspre;
-    double y = P - 0.01 * p.frspre;
-    double prelim = 0. < y ? 0. : y;
+    const double P = COARSE ? FLD(b, FF_P)[n] : pd + p.frspre;
+    const double y = P - 0.01 * p.frspre;
+    const double prelim = 0. < y ? 0. : y;
     FLD(b, FF_P)[n] = P - prelim;
     FLD(b, FF_PDIFF)[n] = pd - prelim;
 }
@@ -3970,8 +3915,7 @@ struct BlockRec {
     void *sw_mem = nullptr;
     size_t nhalo = 0;          // halo slot words
     size_t ntile_slots = 0;    // words of the (J,K)-tile forms' slots (J faces, then K faces)
-    double *kw_scr = nullptr;  // k-omega: per-workgroup maxima of SEPS and their maximum
-    int kw_parts = 0;
+    double *kw_scr = nullptr;  // k-omega: the maximum of SEPS
     int level = 0;             // multigrid level M the slab was registered as
     WallRec walls;
     SweepSt st{};              // staged records of the (J,K)-tile sweeps (allocated on first use)
@@ -4252,8 +4196,7 @@ static int sweep_alloc(ff_ctx *c, BlockRec &r)
     sk.hj = sk.hi + nhi2;
     HIPCHK(c, hipMemsetAsync(r.sw_mem, 0, head * sizeof(unsigned long long), c->stream));
     if (c->prm.iturb == 6) {
-        r.kw_parts = (b.ntot + 255) / 256;
-        if (hipMalloc(&r.kw_scr, sizeof(double) * (size_t)(r.kw_parts + 1)) != hipSuccess)
+        if (hipMalloc(&r.kw_scr, sizeof(double)) != hipSuccess)
             return fail(c, FF_E_NOMEM, "k-omega reduction scratch%s");
     }
     size_t nh = r.nhalo;
@@ -4646,15 +4589,21 @@ static int reflec_impl(ff_ctx *c, BlockRec *r, int level);
 
 // STATIM(M,N,INN,.TRUE.): the state, then REFLEC over the block level's boundary patches
 // (ns3c.f:10497-10512)
+static int state_impl(ff_ctx *c, BlockRec *r, int level, bool save)
+{
+    c->lev = level;
+    int rc = launch(c, "k_state", save ? k_state<true> : k_state<false>, all_grid(r->dev), dim3(256),
+                    make_prm(&c->prm, level), r->dev, save ? r->bc_icyc : (int *)nullptr);
+    if (rc) return rc;
+    return reflec_impl(c, r, level);
+}
+
 int ff_state(ff_ctx *c, int level, int block)
 {
     if (!c) return FF_E_ARG;
     BlockRec *r = find(c, level, block);
     if (!r) return fail(c, FF_E_STATE, "block not registered%s");
-    c->lev = level;
-    int rc = launch(c, "k_state", k_state, all_grid(r->dev), dim3(256), make_prm(&c->prm, level), r->dev);
-    if (rc) return rc;
-    return reflec_impl(c, r, level);
+    return state_impl(c, r, level, false);
 }
 
 int ff_turb(ff_ctx *c, int level, int block)
@@ -4806,10 +4755,7 @@ static int residual_impl(ff_ctx *c, BlockRec *r, int level, int m2, double *resi
     if (c->prm.iturb == 6 && m2 >= 2) {
         // RESIKE's own DERFUN (res3c.f:3749-3769), EXTEND on coarse levels
         const int g0 = level == 1 ? 1 : 0;
-        if ((rc = launch(c, "k_grad_zero", k_grad_zero, all_grid(b), dim3(256), b))) return rc;
-        dim3 g((b.imax + 2 * g0 + 255) / 256, b.jmax + 2 * g0, b.kmax + 2 * g0);
-        if ((rc = launch(c, "k_derfun", k_derfun, g, dim3(256), b, g0))) return rc;
-        if (level >= 2 && (rc = launch(c, "k_extend", k_extend, cells_grid(b, 256), dim3(256), b))) return rc;
+        if ((rc = launch(c, "k_derfun", k_gradients, dim3((b.is + 255) / 256, b.js, b.ks), dim3(256), b, g0))) return rc;
     }
     const bool kw = c->prm.iturb == 6;
     const int nq = kw ? 7 : 5;
@@ -4870,19 +4816,19 @@ static int residual_impl(ff_ctx *c, BlockRec *r, int level, int m2, double *resi
     };
     // ZEROZZ of DRO..DE (DRK, DEPS) on every cell (res3c.f:194-198, 3668-3674): ghost
     // residuals stay zero
-    if ((rc = launch(c, "k_zero", k_zero, all_grid(b), dim3(256), b, nq))) return rc;
+    // (the k-omega form's rounding pass zeroes them on its way)
+    if (!kw && (rc = launch(c, "k_zero", k_zero, all_grid(b), dim3(256), b, nq))) return rc;
     const bool vl = c->prm.iflux == 0;
     if (kw) {
         if (c->residual_mode != FF_RESIDUAL_TILES)
             return fail(c, FF_E_UNSUP, "the k-omega residual has the tile form only%s");
         Prm kp = make_prm(&c->prm, level);
         // CROSKO, its rounding of RK/REPS, FUN1KO's floor, FUN1KO + PRODKE (res3c.f:3817-3994)
-        if ((rc = launch(c, "k_crosko", k_crosko, cells_grid(b, 256), dim3(256), kp, b))) return rc;
-        if ((rc = launch(c, "k_kw_round", k_kw_round, dim3(r->kw_parts), dim3(256), b, r->kw_scr))) return rc;
-        if ((rc = launch(c, "k_max_final", k_max_final, dim3(1), dim3(256), (const double *)r->kw_scr,
-                         r->kw_parts, r->kw_scr + r->kw_parts))) return rc;
-        if ((rc = launch(c, "k_fun1_prod", k_fun1_prod, cells_grid(b, 256), dim3(256), kp, b,
-                         (const double *)(r->kw_scr + r->kw_parts)))) return rc;
+        if ((rc = launch(c, "k_crosko", k_crosko, cells_grid(b, 256), dim3(256), kp, b, r->kw_scr)) ||
+            (rc = launch(c, "k_kw_round", k_kw_round, all_grid(b), dim3(256), b, r->kw_scr)) ||
+            (rc = launch(c, "k_fun1_prod", k_fun1_prod, cells_grid(b, 256), dim3(256), kp, b,
+                         (const double *)r->kw_scr)))
+            return rc;
         if (fns && (rc = gradients())) return rc;
         if ((rc = walls())) return rc;
         if (level == 1 && (rc = inlout_impl(c, r, level))) return rc;
@@ -4979,8 +4925,7 @@ int ff_residual_noalloc(ff_ctx *c, int level, const ff_block *dev, int m2, doubl
     r.level = level;
     r.dev = make_blk(dev);
     if (c->prm.iturb == 6) {
-        r.kw_parts = (r.dev.ntot + 255) / 256;
-        if (r.kw_parts > NA_KW_PARTS)
+        if ((r.dev.ntot + 255) / 256 > NA_KW_PARTS)
             return fail(c, FF_E_ARG, "ff_residual_noalloc: the k-omega residual takes blocks of at most "
                         "8388608 entries including ghost layers (this one has %s)",
                         std::to_string(r.dev.ntot).c_str());
@@ -5128,13 +5073,9 @@ static int update_impl(ff_ctx *c, BlockRec *r, int level)
     const Blk &b = r->dev;
     c->lev = level;
     const bool kw = c->prm.iturb == 6;
-    int rc = kw ? launch(c, "k_fin", k_fin_kw, cells_grid(b, 256), dim3(256), b)
-                : launch(c, "k_fin", k_fin, cells_grid(b, 256), dim3(256), b);
-    if (rc) return rc;
-    if (level >= 2)
-        return launch(c, "k_limits_mg", k_limits_mg, all_grid(b), dim3(256), make_prm(&c->prm, level),
-                      b, 1, kw ? 1 : 0);
-    return launch(c, "k_limits", k_limits, all_grid(b), dim3(256), make_prm(&c->prm, level), b);
+    auto kern = level >= 2 ? (kw ? k_fin<true, true> : k_fin<false, true>)
+                           : (kw ? k_fin<true, false> : k_fin<false, false>);
+    return launch(c, "k_fin", kern, all_grid(b), dim3(256), make_prm(&c->prm, level), b);
 }
 
 // TRANSF/TRANKE from level m to level m+1 of a block (multi.f:156-620)
@@ -5142,21 +5083,9 @@ static int restrict_impl(ff_ctx *c, BlockRec *fr, BlockRec *cr)
 {
     const Blk &f = fr->dev, &cb = cr->dev;
     const bool kw = c->prm.iturb == 6;
-    int rc;
     c->lev = cr->level;
-    dim3 g((cb.imax + 2 + 255) / 256, cb.jmax + 2, cb.kmax + 2);
-    rc = kw ? launch(c, "k_restrict", k_restrict<true>, g, dim3(256), f, cb)
-            : launch(c, "k_restrict", k_restrict<false>, g, dim3(256), f, cb);
-    if (rc) return rc;
-    const int na[3] = {cb.jmax + 4, cb.imax + 4, cb.imax + 4};
-    const int nb[3] = {cb.kmax + 4, cb.kmax + 4, cb.jmax + 4};
-    for (int face = 0; face < 3; face++) {
-        dim3 gg((na[face] + 255) / 256, nb[face]);
-        rc = kw ? launch(c, "k_restrict_ghosts", k_restrict_ghosts<true>, gg, dim3(256), cb, face)
-                : launch(c, "k_restrict_ghosts", k_restrict_ghosts<false>, gg, dim3(256), cb, face);
-        if (rc) return rc;
-    }
-    return FF_OK;
+    return launch(c, "k_restrict", kw ? k_restrict<true> : k_restrict<false>,
+                  dim3((cb.is + 255) / 256, cb.js, cb.ks), dim3(256), f, cb);
 }
 
 static int forcing_impl(ff_ctx *c, BlockRec *r, int phase)
@@ -5173,10 +5102,8 @@ static int prolong_impl(ff_ctx *c, BlockRec *cr, BlockRec *fr, int level_fine)
     const bool kw = c->prm.iturb == 6;
     Prm kp = make_prm(&c->prm, level_fine);
     c->lev = level_fine;
-    int rc = kw ? launch(c, "k_prolong", k_prolong<true>, cells_grid(f, 256), dim3(256), kp, cb, f)
-                : launch(c, "k_prolong", k_prolong<false>, cells_grid(f, 256), dim3(256), kp, cb, f);
-    if (rc) return rc;
-    return launch(c, "k_limits_mg", k_limits_mg, all_grid(f), dim3(256), kp, f, kw ? 1 : 0, kw ? 1 : 0);
+    return launch(c, "k_prolong", kw ? k_prolong<true> : k_prolong<false>,
+                  dim3((f.is + 255) / 256, f.js, f.ks), dim3(256), kp, cb, f);
 }
 
 static int check_pair(ff_ctx *c, BlockRec *fr, BlockRec *cr)
@@ -5206,7 +5133,7 @@ int ff_save_old(ff_ctx *c, int level, int block)
     BlockRec *r = find(c, level, block);
     if (!r) return fail(c, FF_E_STATE, "block not registered%s");
     c->lev = level;
-    return launch(c, "k_save_old", k_save_old, all_grid(r->dev), dim3(256), r->dev, (int *)nullptr);
+    return launch(c, "k_save_old", k_save_old, all_grid(r->dev), dim3(256), r->dev);
 }
 
 int ff_cycle(ff_ctx *c, int block, int ncycles, double *resi)
@@ -5217,9 +5144,7 @@ int ff_cycle(ff_ctx *c, int block, int ncycles, double *resi)
     int rc;
     for (int it = 0; it < ncycles; it++) {
         bool last = it == ncycles - 1;
-        c->lev = 1;
-        if ((rc = launch(c, "k_save_old", k_save_old, all_grid(r->dev), dim3(256), r->dev, r->bc_icyc))) return rc;
-        if ((rc = ff_state(c, 1, block))) return rc;
+        if ((rc = state_impl(c, r, 1, true))) return rc;
         if ((rc = ff_turb(c, 1, block))) return rc;
         if ((rc = residual_impl(c, r, 1, 1, last ? resi : nullptr))) return rc;
         if ((rc = implicit_impl(c, r, 1, true))) return rc;
@@ -5262,9 +5187,7 @@ static int vcycle_once(ff_ctx *c, const std::vector<BlockRec *> &lv, int nlev, i
     int rc;
     BlockRec *r1 = lv[0];
     // level 1: CYCLES ns3c.f:1450-1596
-    c->lev = 1;
-    if ((rc = launch(c, "k_save_old", k_save_old, all_grid(r1->dev), dim3(256), r1->dev, r1->bc_icyc))) return rc;
-    if ((rc = ff_state(c, 1, block))) return rc;
+    if ((rc = state_impl(c, r1, 1, true))) return rc;
     if ((rc = ff_turb(c, 1, block))) return rc;
     if ((rc = residual_impl(c, r1, 1, 1, rs, rb, host))) return rc;
     if ((rc = implicit_impl(c, r1, 1, true))) return rc;
@@ -5278,8 +5201,7 @@ static int vcycle_once(ff_ctx *c, const std::vector<BlockRec *> &lv, int nlev, i
         if ((rc = restrict_impl(c, fr, cr))) return rc;
         if ((rc = ff_state(c, m, block))) return rc;
         if ((rc = residual_impl(c, cr, m, m, nullptr))) return rc;
-        if ((rc = forcing_impl(c, cr, 0))) return rc;
-        if ((rc = forcing_impl(c, cr, 1))) return rc;
+        if ((rc = forcing_impl(c, cr, 2))) return rc;
         if ((rc = implicit_impl(c, cr, m, true))) return rc;
         if ((rc = update_impl(c, cr, m))) return rc;
     }
