@@ -6,7 +6,7 @@
 // backward pass PRED (imps4.f:788-905; k-omega PREDKE imps4.f:2084-2229), a pointwise
 // diagonal DIAG (imps4.f:911-971; DIAGKE imps4.f:2235-2309) and a forward pass CORR
 // (imps4.f:671-787; CORRKE imps4.f:1939-2078).  Each pass is a recurrence along one grid
-// line only, so the lines are independent: a thread owns one line and marches along it.
+// line only, so the lines are independent.
 // The reference sorts its arrays so that the swept direction runs slowest (SORT38, SORTZZ
 // of multi.f: IJK for K, JKI for I, KIJ for J) and loops over the entries of its sorted
 // (a, b) plane from entry IN+1 of the first interior row to the end of the last (DO I =
@@ -92,16 +92,16 @@ __device__ __forceinline__ void sym1ke(double x[7], const double w[7], double rk
     x[3] = a2z * x2i + a23 * x3i + a33 * x4i;
 }
 
-// The sweep's line of thread t, as the flat offset of its cell m = 1 minus one step: the
-// reference's plane entry f = IN + t*step on the K and I sweeps (consecutive threads take
-// neighbouring I columns on the K sweep; on the I sweep each thread walks its own
-// contiguous row); on the J sweep the entries are renumbered with the middle index b (= I)
-// fastest so that consecutive threads again take neighbouring I columns.  The set of
-// entries is the reference's: f = a + b*(NA+4) >= IN, every 2*IN+1-th with NA = 1.
-__device__ __forceinline__ bool dd_line(const DdDir &r, int dir, int t, int &base)
+// The sweep's line t, as the flat offset of its cell m = 1 minus one step: the reference's
+// plane entry f = IN + t*step on the K and I sweeps (consecutive lines are neighbouring I
+// columns on the K sweep, rows on the I sweep); on the J sweep the entries are renumbered with the middle index b (= I)
+// fastest so that consecutive lines again take neighbouring I columns.  The set of
+// entries is the reference's: f = a + b*(NA+4) >= IN, every 2*IN+1-th with NA = 1.  a0: the
+// line's fast index.
+__device__ __forceinline__ bool dd_line(const DdDir &r, int dir, int t, int &base, int &a0)
 {
     const int ist = r.na + 2 * FF_GHOST;
-    int a0, b0;
+    int b0;
     if (dir == 2) {
         b0 = t % r.nb;
         a0 = t / r.nb;
@@ -117,7 +117,7 @@ __device__ __forceinline__ bool dd_line(const DdDir &r, int dir, int t, int &bas
     return true;
 }
 
-// threads of a sweep launch
+// line numbers of a sweep launch
 static int dd_threads(const DdDir &r, int dir)
 {
     return dir == 2 ? (r.na + 2 * FF_GHOST) * r.nb : dd_lines(r);
@@ -130,7 +130,7 @@ static int dd_threads(const DdDir &r, int dir)
 // characteristic variables it uses (PRED: the lower face, CORR: the upper face).
 struct DdIn {
     double dt1, vol, voln, u, v, w, c, ro, ron, vis, vist, visn, vistn;
-    double aflux, adiag, fx, fy, fz;
+    double aflux, adiag, fx, fy, fz, lx, ly, lz;   // l: the other face's normal (DIAG)
     double d[7], rk, drdp, drdh;
 };
 
@@ -156,6 +156,11 @@ __device__ __forceinline__ void dd_load(const Prm &p, const Blk &b, const DdDir 
     x.fx = r.AX[nf];
     x.fy = r.AY[nf];
     x.fz = r.AZ[nf];
+    if (FWD) {
+        x.lx = r.AX[n];
+        x.ly = r.AY[n];
+        x.lz = r.AZ[n];
+    }
 #pragma unroll
     for (int q = 0; q < (KE ? 7 : 5); q++) x.d[q] = FLD(b, FF_DRO + q)[n];
     if (KE) {
@@ -165,122 +170,26 @@ __device__ __forceinline__ void dd_load(const Prm &p, const Blk &b, const DdDir 
     }
 }
 
-// PRED (FWD = false: backward along the line) or CORR (FWD = true: forward) along every line
-// of one direction.  The reads of the next cell are issued before the current cell's
-// arithmetic (they do not depend on the recurrence), so their latency overlaps it.
-template <bool KE, bool FWD>
-__global__ void __launch_bounds__(128) k_ddadi_sweep(Prm p, Blk b, DdDir r, int dir, int nthreads)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    int base;
-    if (t >= nthreads || !dd_line(r, dir, t, base)) return;
-    constexpr int NV = KE ? 7 : 5;
-    double *D[7] = {FLD(b, FF_DRO), FLD(b, FF_DM), FLD(b, FF_DN), FLD(b, FF_DW), FLD(b, FF_DE),
-                    FLD(b, FF_DRK), FLD(b, FF_DEPS)};
-    const double cdiff = 2., dturb = 1., vrel = 1.E-21;
-    double bd[7] = {0., 0., 0., 0., 0., 0., 0.};
-    int m = FWD ? 1 : r.nm;
-    DdIn cur, nxt;
-    dd_load<KE, FWD>(p, b, r, base + m * r.sm, cur);
-    for (int s = 0; s < r.nm; s++) {
-        const int n = base + m * r.sm;
-        const int mn = FWD ? m + 1 : m - 1;
-        if (s + 1 < r.nm) dd_load<KE, FWD>(p, b, r, base + mn * r.sm, nxt);
-        double x[7], y[7], a21, a22, a23, a31, a32, a33;
-#pragma unroll
-        for (int q = 0; q < 5; q++) x[q] = cur.dt1 * cur.aflux * bd[q] + cur.vol * cur.d[q];
-        if (KE) {
-#pragma unroll
-            for (int q = 5; q < 7; q++) x[q] = dturb * cur.dt1 * cur.aflux * bd[q] + cur.vol * cur.d[q];
-            syike(y, x, cur.c, cur.ro, cur.fx, cur.fy, cur.fz, a21, a22, a23, a31, a32, a33);
-        } else {
-            syi(y[0], y[1], y[2], y[3], y[4], x[0], x[1], x[2], x[3], x[4], cur.c, cur.ro, cur.fx,
-                cur.fy, cur.fz, a21, a22, a23, a31, a32, a33);
-        }
-        const double rl1 = cur.fx * cur.u + cur.fy * cur.v + cur.fz * cur.w - 0.;
-        const double rl2 = rl1 + cur.c, rl5 = rl1 - cur.c;
-        const double ff = FWD ? .5 : (m == 1 ? .25 : .5);
-        const double rnum = ff * (cur.vol + cur.voln) * (cur.ro + cur.ron);
-        const double tt = cdiff * cur.adiag / rnum * (cur.vist + cur.vis + cur.vistn + cur.visn);
-        double x1, x2, x5;
-        if (FWD) {
-            x1 = dmax(rl1, 0.) + tt; x2 = dmax(rl2, 0.) + tt; x5 = dmax(rl5, 0.) + tt;
-        } else {
-            x1 = dmax(-rl1, 0.) + tt; x2 = dmax(-rl2, 0.) + tt; x5 = dmax(-rl5, 0.) + tt;
-        }
-        const double x1a = fabs(rl1) + tt, x2a = fabs(rl2) + tt, x5a = fabs(rl5) + tt;
-        const double xa[5] = {x1a, x2a, x1a, x1a, x5a};
-        if (KE) {
-#pragma unroll
-            for (int q = 0; q < 5; q++) y[q] = y[q] / (cur.vol + vrel + cur.dt1 * xa[q] * cur.adiag);
-#pragma unroll
-            for (int q = 5; q < 7; q++) y[q] = y[q] / (cur.vol + vrel + dturb * cur.dt1 * (x1a * cur.adiag + 0.));
-            double o[7];
-            sym1ke(o, y, cur.rk, cur.c, cur.ro, cur.drdp, cur.drdh, cur.fx, cur.fy, cur.fz, a21, a22,
-                   a23, a31, a32, a33);
-#pragma unroll
-            for (int q = 0; q < 7; q++) D[q][n] = o[q];
-        } else {
-#pragma unroll
-            for (int q = 0; q < 5; q++) y[q] = y[q] / (cur.vol + cur.dt1 * xa[q] * cur.adiag);
-            double o0, o1, o2, o3, o4;
-            sym1i(o0, o1, o2, o3, o4, y[0], y[1], y[2], y[3], y[4], cur.c, cur.ro, cur.fx, cur.fy,
-                  cur.fz, a21, a22, a23, a31, a32, a33);
-            D[0][n] = o0; D[1][n] = o1; D[2][n] = o2; D[3][n] = o3; D[4][n] = o4;
-        }
-        // the flux handed to the next cell of the line
-        const double xs[7] = {x1, x2, x1, x1, x5, x1, x1};
-#pragma unroll
-        for (int q = 0; q < NV; q++) y[q] = xs[q] * y[q];
-        if (KE)
-            sym1ke(bd, y, cur.rk, cur.c, cur.ro, cur.drdp, cur.drdh, cur.fx, cur.fy, cur.fz, a21, a22,
-                   a23, a31, a32, a33);
-        else
-            sym1i(bd[0], bd[1], bd[2], bd[3], bd[4], y[0], y[1], y[2], y[3], y[4], cur.c, cur.ro,
-                  cur.fx, cur.fy, cur.fz, a21, a22, a23, a31, a32, a33);
-        cur = nxt;
-        m = mn;
-    }
-}
-
-// DIAG (DIAGKE) on every entry of the direction's plane and line, one thread each: x runs
-// along I (stride 1), y and z over the other two sorted indices
+// DIAG (DIAGKE) of a cell, on the operands CORR reads of it
 template <bool KE>
-__global__ void __launch_bounds__(256) k_ddadi_diag(Prm p, Blk b, DdDir r, int dir)
+__device__ __forceinline__ void dd_diag(const DdIn &x, double d[7])
 {
-    const int gx = blockIdx.x * blockDim.x + threadIdx.x, gy = blockIdx.y, gz = blockIdx.z;
-    int a0, b0, m;
-    if (dir == 0) { a0 = gx; b0 = gy; m = gz + 1; }      // a = I, b = J, m = K
-    else if (dir == 1) { m = gx + 1; a0 = gy; b0 = gz; } // a = J, b = K, m = I
-    else { b0 = gx; a0 = gy; m = gz + 1; }                // a = K, b = I, m = J
-    const int ist = r.na + 2 * FF_GHOST;
-    if (a0 >= ist || b0 >= r.nb || m > r.nm) return;
-    if ((b0 == 0 && a0 < FF_GHOST) || (r.na == 1 && a0 != FF_GHOST)) return;
-    const int n = a0 * r.sa + (b0 + FF_GHOST) * r.sb + (m + FF_GHOST - 1) * r.sm, nu = n + r.sm;
-    double *D[7] = {FLD(b, FF_DRO), FLD(b, FF_DM), FLD(b, FF_DN), FLD(b, FF_DW), FLD(b, FF_DE),
-                    FLD(b, FF_DRK), FLD(b, FF_DEPS)};
-    const double *vol = FLD(b, FF_VOL), *u = FLD(b, FF_U), *v = FLD(b, FF_V), *w = FLD(b, FF_W),
-                 *c = FLD(b, FF_C), *ro = FLD(b, FF_RO);
     const double dturb = 1.;
-    const double dt1 = p.theta * FLD(b, FF_DTL)[n];
-    const double fx = r.AX[nu], fy = r.AY[nu], fz = r.AZ[nu];
-    double xv[7], y[7], a21, a22, a23, a31, a32, a33;
-#pragma unroll
-    for (int q = 0; q < (KE ? 7 : 5); q++) xv[q] = D[q][n];
+    double y[7], a21, a22, a23, a31, a32, a33;
     if (KE)
-        syike(y, xv, c[n], ro[n], fx, fy, fz, a21, a22, a23, a31, a32, a33);
+        syike(y, x.d, x.c, x.ro, x.fx, x.fy, x.fz, a21, a22, a23, a31, a32, a33);
     else
-        syi(y[0], y[1], y[2], y[3], y[4], xv[0], xv[1], xv[2], xv[3], xv[4], c[n], ro[n], fx, fy, fz,
-            a21, a22, a23, a31, a32, a33);
-    double ucon = fx * u[n] + fy * v[n] + fz * w[n] - 0.;
-    const double rl2n = dmax(-(ucon + c[n]), 0.), rl5n = dmax(-(ucon - c[n]), 0.);
+        syi(y[0], y[1], y[2], y[3], y[4], x.d[0], x.d[1], x.d[2], x.d[3], x.d[4], x.c, x.ro, x.fx, x.fy,
+            x.fz, a21, a22, a23, a31, a32, a33);
+    double ucon = x.fx * x.u + x.fy * x.v + x.fz * x.w - 0.;
+    const double rl2n = dmax(-(ucon + x.c), 0.), rl5n = dmax(-(ucon - x.c), 0.);
     const double rl1n = dmax(-ucon, 0.);
-    ucon = r.AX[n] * u[n] + r.AY[n] * v[n] + r.AZ[n] * w[n] - 0.;
-    const double rl2p = dmax(ucon + c[n], 0.), rl5p = dmax(ucon - c[n], 0.);
+    ucon = x.lx * x.u + x.ly * x.v + x.lz * x.w - 0.;
+    const double rl2p = dmax(ucon + x.c, 0.), rl5p = dmax(ucon - x.c, 0.);
     const double rl1p = dmax(ucon, 0.);
-    const double dt = KE ? dt1 / (vol[n] + 1.E-21) : dt1 / vol[n];
-    const double s1 = r.A[n] * rl1p + r.A[nu] * rl1n, s2 = r.A[n] * rl2p + r.A[nu] * rl2n;
-    const double s5 = r.A[n] * rl5p + r.A[nu] * rl5n;
+    const double dt = KE ? x.dt1 / (x.vol + 1.E-21) : x.dt1 / x.vol;
+    const double s1 = x.aflux * rl1p + x.adiag * rl1n, s2 = x.aflux * rl2p + x.adiag * rl2n;
+    const double s5 = x.aflux * rl5p + x.adiag * rl5n;
     y[0] = y[0] * (1. + dt * s1);
     y[1] = y[1] * (1. + dt * s2);
     y[2] = y[2] * (1. + dt * s1);
@@ -289,61 +198,304 @@ __global__ void __launch_bounds__(256) k_ddadi_diag(Prm p, Blk b, DdDir r, int d
     if (KE) {
         y[5] = y[5] * (1. + dturb * dt * (s1 + 0.));
         y[6] = y[6] * (1. + dturb * dt * (s1 + 0.));
-        double o[7];
-        sym1ke(o, y, FLD(b, FF_RK)[n], c[n], ro[n], FLD(b, FF_DRDP)[n], FLD(b, FF_DRDH)[n], fx, fy,
-               fz, a21, a22, a23, a31, a32, a33);
-#pragma unroll
-        for (int q = 0; q < 7; q++) D[q][n] = o[q];
+        sym1ke(d, y, x.rk, x.c, x.ro, x.drdp, x.drdh, x.fx, x.fy, x.fz, a21, a22, a23, a31, a32, a33);
     } else {
-        double o0, o1, o2, o3, o4;
-        sym1i(o0, o1, o2, o3, o4, y[0], y[1], y[2], y[3], y[4], c[n], ro[n], fx, fy, fz, a21, a22,
-              a23, a31, a32, a33);
-        D[0][n] = o0; D[1][n] = o1; D[2][n] = o2; D[3][n] = o3; D[4][n] = o4;
+        sym1i(d[0], d[1], d[2], d[3], d[4], y[0], y[1], y[2], y[3], y[4], x.c, x.ro, x.fx, x.fy, x.fz,
+              a21, a22, a23, a31, a32, a33);
     }
 }
 
-// the end of IMPS on the interior cells: dh -> dT (DIVV12 imps3.f:483) and, with the
-// k-omega model, D(rho k), D(rho omega) times RO (MULV12 imps3.f:497-500)
+// The recurrence of a line needs of each cell only values that do not depend on it (VOL*D,
+// DT1*A, the face's basis, the scalars of SYI and SYM1I, the denominators, the eigenvalues):
+// a record of them per cell, in LDS.  VD holds the quotients Y after the march.
 template <bool KE>
-__global__ void __launch_bounds__(256) k_ddadi_end(Blk b)
+struct DdRec {
+    static constexpr int NV = KE ? 7 : 5, ND = KE ? 4 : 3;   // ND: denominators X1, X2, X5 (, K)
+    static constexpr int VD = 0, M = NV, N = M + 1, T1 = N + 3, T2 = T1 + 3, ROC = T2 + 3, YP = ROC + 1,
+                         PROC = YP + 1, SC = PROC + 1,       // KE: YDRP, DRH*RO, .667*RO; else RO
+                         DEN = SC + (KE ? 3 : 1), REC = DEN + ND, X = REC + ND, NF = X + 3;
+    static_assert(NF % 2 == 0, "the record is read in pairs");
+};
+
+// Lines and steps of a line per LDS buffer, and the waves that fill it
+constexpr int DD_L = 32, DD_CH = 8, DD_PW = DD_L * DD_CH / 64;
+
+// doubles of a step's records: pairs of fields, [pair][line][2], and 32 bytes so that the steps of
+// one line (the I sweep's waves hold 8 of each line) fall in different banks
+template <bool KE>
+constexpr int dd_slot() { return DdRec<KE>::NF * DD_L + 4; }
+
+typedef double dd2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ dd2 *dd_pair(double *rec, int q) { return (dd2 *)(rec + q * 2 * DD_L); }
+
+// |x| in 2^-460 .. 2^460: the exponent's distance from the lower end (large for zero, infinity
+// and NaN too)
+__device__ __forceinline__ unsigned dd_mag(double x)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1, j = blockIdx.y + 1, k = blockIdx.z + 1;
-    if (i > b.imax) return;
-    const int n = cid(b, i, j, k);
-    FLD(b, FF_DRO)[n] = FLD(b, FF_DRO)[n] / FLD(b, FF_CP)[n];
-    if (KE) {
-        FLD(b, FF_DRK)[n] = FLD(b, FF_DRK)[n] * FLD(b, FF_RO)[n];
-        FLD(b, FF_DEPS)[n] = FLD(b, FF_DEPS)[n] * FLD(b, FF_RO)[n];
-    }
+    return ((unsigned)((unsigned long long)__double_as_longlong(x) >> 32) << 1) - (563u << 21);
+}
+constexpr unsigned DD_MAG = 920u << 21;
+
+// y/d, correctly rounded, from r = 1/d correctly rounded: two corrections of y*r with exact
+// remainders (Markstein, IBM J. Res. Dev. 34, 1990).  Holds for d and the quotient in
+// dd_mag's range, where no remainder underflows; the caller divides otherwise.  Five operations for
+// a division's fifteen, on the march's chain.
+__device__ __forceinline__ double dd_quot(double y, double d, double r)
+{
+    double q = y * r;
+    q = fma(fma(-q, d, y), r, q);
+    return fma(fma(-q, d, y), r, q);
 }
 
-// the three DDADI directions in IMPS's order, K, I, J, each PRED, DIAG, CORR, then the end
-// of IMPS
+// a denominator and its reciprocal, NaN where dd_quot does not hold
+__device__ __forceinline__ double dd_recip(double d)
+{
+    return dd_mag(d) < DD_MAG ? 1. / d : __longlong_as_double(0x7ff8000000000000LL);
+}
+
+// SYM1I / SYM1KE with a record's values
+template <bool KE>
+__device__ __forceinline__ void dd_sym1(const double *f, const double *w, double *x)
+{
+    using R = DdRec<KE>;
+    const double pc2 = .5 * f[R::YP];
+    x[0] = w[0] + pc2 * (w[1] + w[4]);
+    const double x2i = f[R::PROC] * (w[1] - w[4]);
+    double x5 = .5 * (w[1] + w[4]);
+    if (KE) {
+        x5 = f[R::SC] * (x5 - f[R::SC + 1] * x[0] - f[R::SC + 2] * w[5]);
+        x[5] = w[5];
+        x[6] = w[6];
+    }
+    x[4] = x5;
+#pragma unroll
+    for (int q = 0; q < 3; q++) x[1 + q] = f[R::N + q] * x2i + f[R::T1 + q] * w[2] + f[R::T2 + q] * w[3];
+}
+
+// the record of a cell (m: its place on the line) to LDS
+template <bool KE, bool FWD>
+__device__ __forceinline__ void dd_record(const DdIn &x, int m, double *rec)
+{
+    using R = DdRec<KE>;
+    const double cdiff = 2., dturb = 1., vrel = 1.E-21;
+    double f[R::NF], d[7];
+    if (FWD) {
+        dd_diag<KE>(x, d);
+    } else {
+#pragma unroll
+        for (int q = 0; q < R::NV; q++) d[q] = x.d[q];
+    }
+#pragma unroll
+    for (int q = 0; q < R::NV; q++) f[R::VD + q] = x.vol * d[q];
+    f[R::M] = x.dt1 * x.aflux;
+    f[R::N] = x.fx; f[R::N + 1] = x.fy; f[R::N + 2] = x.fz;
+    surfvects(x.fx, x.fy, x.fz, f[R::T1], f[R::T1 + 1], f[R::T1 + 2], f[R::T2], f[R::T2 + 1], f[R::T2 + 2]);
+    const double ypro = 1. / x.ro, pc2 = .5 * ypro;
+    f[R::ROC] = x.ro * x.c;
+    f[R::YP] = ypro;
+    f[R::PROC] = pc2 / x.c;
+    const double rl1 = x.fx * x.u + x.fy * x.v + x.fz * x.w - 0.;
+    const double rl2 = rl1 + x.c, rl5 = rl1 - x.c;
+    const double ff = FWD ? .5 : (m == 1 ? .25 : .5);
+    const double rnum = ff * (x.vol + x.voln) * (x.ro + x.ron);
+    const double tt = cdiff * x.adiag / rnum * (x.vist + x.vis + x.vistn + x.visn);
+    if (FWD) {
+        f[R::X] = dmax(rl1, 0.) + tt; f[R::X + 1] = dmax(rl2, 0.) + tt; f[R::X + 2] = dmax(rl5, 0.) + tt;
+    } else {
+        f[R::X] = dmax(-rl1, 0.) + tt; f[R::X + 1] = dmax(-rl2, 0.) + tt; f[R::X + 2] = dmax(-rl5, 0.) + tt;
+    }
+    const double xa[3] = {fabs(rl1) + tt, fabs(rl2) + tt, fabs(rl5) + tt};
+    if (KE) {
+        const double drh = .667 * x.rk * (ypro * ypro) * x.drdh;
+        f[R::SC] = 1. / (1. + .667 * x.rk * ypro * x.drdp);
+        f[R::SC + 1] = drh * x.ro;
+        f[R::SC + 2] = .667 * x.ro;
+#pragma unroll
+        for (int q = 0; q < 3; q++) f[R::DEN + q] = x.vol + vrel + x.dt1 * xa[q] * x.adiag;
+        f[R::DEN + R::ND - 1] = x.vol + vrel + dturb * x.dt1 * (xa[0] * x.adiag + 0.);
+    } else {
+        f[R::SC] = x.ro;
+#pragma unroll
+        for (int q = 0; q < 3; q++) f[R::DEN + q] = x.vol + x.dt1 * xa[q] * x.adiag;
+    }
+#pragma unroll
+    for (int q = 0; q < R::ND; q++) f[R::REC + q] = dd_recip(f[R::DEN + q]);
+#pragma unroll
+    for (int q = 0; q < R::NF / 2; q++) *dd_pair(rec, q) = dd2{f[2 * q], f[2 * q + 1]};
+}
+
+// PRED (FWD = false: backward along the line) or DIAG and CORR (FWD = true: forward) along
+// every line of one direction; last: the end of IMPS on the interior cells as well, dh -> dT
+// (DIVV12 imps3.f:483) and, with the k-omega model, D(rho k), D(rho omega) times RO (MULV12
+// imps3.f:497-500).
+//
+// A line is a serial chain, and there are too few lines to fill the chip (96x72x50: 59 waves
+// on the I sweep), so what counts is the time of one step.  Wave 0 of a workgroup marches 32
+// lines from records in LDS: SYI, the quotients, the flux to the next cell, nothing else.
+// The other four waves work a buffer of 8 steps ahead and one behind: they load the cells,
+// form the records (two thirds of the arithmetic, with the square root and all divisions but
+// the quotients') and, from the quotients the march left, the cells' increments.  On the I
+// sweep a wave takes 8 steps of 8 lines, so that a load touches 8 runs of 64 bytes instead of
+// 64 cache lines.  k-omega, 96x72x50: PRED 37 to 64 us, DIAG and CORR 37 to 64; with one thread
+// per line doing all of it (and DIAG a pass of its own) the six sweeps took 910 us, 290 each on
+// the I sweep, and the stage 1335 us against 538.
+template <bool KE, bool FWD>
+__global__ void __launch_bounds__((1 + DD_PW) * 64) k_ddadi_sweep(Prm p, Blk b, DdDir r, int dir, int nlines,
+                                                                   int last)
+{
+    using R = DdRec<KE>;
+    __shared__ __align__(16) double buf[2][DD_CH * dd_slot<KE>()];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x / 64;
+    const int nch = (r.nm + DD_CH - 1) / DD_CH;
+    if (wv == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        int base, a0;
+        const int t = blockIdx.x * DD_L + lane;
+        const bool on = lane < DD_L && t < nlines && dd_line(r, dir, t, base, a0);
+        double bd[7] = {0., 0., 0., 0., 0., 0., 0.};
+        lds_step_barrier();
+        for (int c = 0; c < nch; c++) {
+            if (on) {
+                double *const rec = buf[c & 1] + lane * 2;
+                const int cnt = min(DD_CH, r.nm - c * DD_CH);
+                double f[2][R::NF];
+                auto read = [&](int s, double *g) {
+#pragma unroll
+                    for (int q = 0; q < R::NF / 2; q++) {
+                        const dd2 v = *dd_pair(rec + s * dd_slot<KE>(), q);
+                        g[2 * q] = v.x;
+                        g[2 * q + 1] = v.y;
+                    }
+                };
+                read(0, f[0]);
+#pragma unroll
+                for (int s = 0; s < DD_CH; s++) {
+                    if (s >= cnt) break;
+                    const double *g = f[s & 1];
+                    // (past the last step of a line: a slot of the same buffer, not used)
+                    if (s + 1 < DD_CH) read(s + 1, f[(s + 1) & 1]);
+                    double x[7], y[7], z[7];
+#pragma unroll
+                    for (int q = 0; q < R::NV; q++) x[q] = g[R::M] * bd[q] + g[R::VD + q];
+                    const double z2 = g[R::N] * x[1] + g[R::N + 1] * x[2] + g[R::N + 2] * x[3];
+                    z[2] = g[R::T1] * x[1] + g[R::T1 + 1] * x[2] + g[R::T1 + 2] * x[3];
+                    z[3] = g[R::T2] * x[1] + g[R::T2 + 1] * x[2] + g[R::T2 + 2] * x[3];
+                    z[1] = g[R::ROC] * z2 + x[4];
+                    z[4] = -g[R::ROC] * z2 + x[4];
+                    if (KE) {
+                        z[0] = x[0] - g[R::YP] * x[4];
+                        z[5] = x[5];
+                        z[6] = x[6];
+                    } else {
+                        double v = dd_quot(x[4], g[R::SC], g[R::YP]);
+                        if (max(dd_mag(v), dd_mag(g[R::SC])) >= DD_MAG) v = x[4] / g[R::SC];
+                        z[0] = x[0] - v;
+                    }
+                    constexpr int dn[7] = {0, 1, 0, 0, 2, R::ND - 1, R::ND - 1};
+                    unsigned mag = 0;
+#pragma unroll
+                    for (int q = 0; q < R::NV; q++) {
+                        y[q] = dd_quot(z[q], g[R::DEN + dn[q]], g[R::REC + dn[q]]);
+                        mag = max(mag, dd_mag(y[q]));
+                    }
+                    if (mag >= DD_MAG) {
+#pragma unroll
+                        for (int q = 0; q < R::NV; q++) y[q] = z[q] / g[R::DEN + dn[q]];
+                    }
+                    double *const o = rec + s * dd_slot<KE>();
+                    *dd_pair(o, 0) = dd2{y[0], y[1]};
+                    *dd_pair(o, 1) = dd2{y[2], y[3]};
+                    if (KE) {
+                        *dd_pair(o, 2) = dd2{y[4], y[5]};
+                        *(double *)dd_pair(o, 3) = y[6];
+                    } else {
+                        *(double *)dd_pair(o, 2) = y[4];
+                    }
+                    // the flux handed to the next cell of the line
+                    constexpr int xs[7] = {0, 1, 0, 0, 2, 0, 0};
+#pragma unroll
+                    for (int q = 0; q < R::NV; q++) y[q] = g[R::X + xs[q]] * y[q];
+                    dd_sym1<KE>(g, y, bd);
+                }
+            }
+            lds_step_barrier();
+        }
+        return;
+    }
+    // this lane's line and its step within each buffer
+    const int w = wv - 1;
+    const int ln = dir == 1 ? w * (64 / DD_CH) + lane / DD_CH : lane % DD_L;
+    const int st = dir == 1 ? lane % DD_CH : w * (64 / DD_L) + lane / DD_L;
+    int base = 0, a0 = 0;
+    const int t = blockIdx.x * DD_L + ln;
+    const bool on = t < nlines && dd_line(r, dir, t, base, a0);
+    double *const rec = buf[0] + st * dd_slot<KE>() + ln * 2;
+    constexpr int BUF = DD_CH * dd_slot<KE>();
+    double *D[7] = {FLD(b, FF_DRO), FLD(b, FF_DM), FLD(b, FF_DN), FLD(b, FF_DW), FLD(b, FF_DE),
+                    FLD(b, FF_DRK), FLD(b, FF_DEPS)};
+    auto cell = [&](int c, int &m) {
+        const int s = c * DD_CH + st;
+        m = FWD ? s + 1 : r.nm - s;
+        return on && c < nch && s < r.nm;
+    };
+    DdIn in;
+    int m;
+    auto fetch = [&](int c) {
+        if (cell(c, m)) dd_load<KE, FWD>(p, b, r, base + m * r.sm, in);
+    };
+    auto fill = [&](int c) {
+        if (cell(c, m)) dd_record<KE, FWD>(in, m, rec + (c & 1) * BUF);
+    };
+    auto finish = [&](int c) {
+        if (!cell(c, m)) return;
+        const int n = base + m * r.sm;
+        double f[R::NF], o[7];
+#pragma unroll
+        for (int q = 0; q < (R::DEN + 1) / 2; q++) {
+            const dd2 v = *dd_pair(rec + (c & 1) * BUF, q);
+            f[2 * q] = v.x;
+            f[2 * q + 1] = v.y;
+        }
+        dd_sym1<KE>(f, f + R::VD, o);
+        if (FWD && last && a0 >= FF_GHOST && a0 < FF_GHOST + r.na) {
+            o[0] = o[0] / FLD(b, FF_CP)[n];
+            if (KE) {
+                o[5] = o[5] * FLD(b, FF_RO)[n];
+                o[6] = o[6] * FLD(b, FF_RO)[n];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < R::NV; q++) D[q][n] = o[q];
+    };
+    fetch(0);
+    fill(0);
+    fetch(1);
+    lds_step_barrier();
+    for (int c = 0; c < nch; c++) {
+        if (c > 0) finish(c - 1);
+        fill(c + 1);
+        fetch(c + 2);
+        lds_step_barrier();
+    }
+    finish(nch - 1);
+}
+
+// the three DDADI directions in IMPS's order, K, I, J, each PRED, then DIAG and CORR; the
+// last with the end of IMPS
 static int ddadi_impl(ff_ctx *c, const Prm &kp, const Blk &b)
 {
     const bool ke = c->prm.iturb == 6;
+    auto pred = ke ? k_ddadi_sweep<true, false> : k_ddadi_sweep<false, false>;
+    auto corr = ke ? k_ddadi_sweep<true, true> : k_ddadi_sweep<false, true>;
     for (int dir = 0; dir < 3; dir++) {
         const DdDir r = dd_dir(b, dir);
         const int nt = dd_threads(r, dir);
-        const dim3 g((unsigned)((nt + 127) / 128)), t(128);
-        // DIAG: x along I, y and z over the other two indices of the sorted order
-        const int ist = r.na + 2 * FF_GHOST;
-        const int xn = dir == 0 ? ist : dir == 1 ? r.nm : r.nb;
-        const dim3 gd((unsigned)((xn + 255) / 256), dir == 0 ? r.nb : ist, dir == 1 ? r.nb : r.nm);
+        const dim3 g((unsigned)((nt + DD_L - 1) / DD_L)), t((1 + DD_PW) * 64);
         int rc;
-        if (ke) {
-            if ((rc = launch(c, "k_ddadi", k_ddadi_sweep<true, false>, g, t, kp, b, r, dir, nt)) ||
-                (rc = launch(c, "k_ddadi", k_ddadi_diag<true>, gd, dim3(256), kp, b, r, dir)) ||
-                (rc = launch(c, "k_ddadi", k_ddadi_sweep<true, true>, g, t, kp, b, r, dir, nt)))
-                return rc;
-        } else {
-            if ((rc = launch(c, "k_ddadi", k_ddadi_sweep<false, false>, g, t, kp, b, r, dir, nt)) ||
-                (rc = launch(c, "k_ddadi", k_ddadi_diag<false>, gd, dim3(256), kp, b, r, dir)) ||
-                (rc = launch(c, "k_ddadi", k_ddadi_sweep<false, true>, g, t, kp, b, r, dir, nt)))
-                return rc;
-        }
+        if ((rc = launch(c, "k_ddadi", pred, g, t, kp, b, r, dir, nt, 0)) ||
+            (rc = launch(c, "k_ddadi", corr, g, t, kp, b, r, dir, nt, dir == 2 ? 1 : 0)))
+            return rc;
     }
-    const dim3 ge((unsigned)((b.imax + 255) / 256), b.jmax, b.kmax);
-    return ke ? launch(c, "k_ddadi_end", k_ddadi_end<true>, ge, dim3(256), b)
-              : launch(c, "k_ddadi_end", k_ddadi_end<false>, ge, dim3(256), b);
+    return FF_OK;
 }
