@@ -2478,8 +2478,14 @@ __device__ __forceinline__ FaceBasis basis_get(const double *v)
 // Both records of every cell: thread (lane, step) of tile blockIdx.x, PSW steps per
 // workgroup, so that a workgroup's loads of a column run along I and its record stores are
 // whole rows.  The records are read back only by the sweeps, long after: non-temporal
-// stores keep them from displacing the caches' working set on the way out.
-constexpr int PSW = 4;             // record-pass steps per workgroup, and waves per workgroup
+// stores keep them from displacing the caches' working set on the way out.  The corrector's
+// operands are loaded with the predictor's, ahead of its stores: one wait for memory, and the
+// operands both records share are read once.  Bound by memory on large blocks (768 bytes
+// of records per cell in FP64: 192x96x96 SST 632 us, of which 366 with the loads left out and
+// 242 with the stores), by latency on small ones.  Two steps per workgroup: 128x64x64 121 us
+// and 101x53x47 74 us against 144 and 85 with four, 149 and 84 with one; 192x96x96 the same
+// with two as with four, 763 with one.
+constexpr int PSW = 2;             // record-pass steps per workgroup, and waves per workgroup
 
 template <bool KE, typename RT = double>
 __global__ void __launch_bounds__(PSW * TW) k_sweep_prep(Prm p, Blk b, Sweep sw, SweepSt st,
@@ -2493,7 +2499,8 @@ __global__ void __launch_bounds__(PSW * TW) k_sweep_prep(Prm p, Blk b, Sweep sw,
     if (tl < 0) return;
     // wave w takes TW/PSW lanes over the workgroup's PSW steps, the steps fastest: the PSW
     // consecutive steps of a lane are PSW consecutive cells along I, so a load instruction
-    // touches TW/PSW short runs instead of TW separate cache lines
+    // touches TW/PSW short runs instead of TW separate cache lines, and the lines come again
+    // from L2 for the steps that follow
     static_assert(TW % PSW == 0, "the lanes of a wave split over the record-pass steps");
     const int li = threadIdx.x % TW;
     const int lane = (TW / PSW) * (int)(threadIdx.x / TW) + li / PSW;
@@ -2505,6 +2512,8 @@ __global__ void __launch_bounds__(PSW * TW) k_sweep_prep(Prm p, Blk b, Sweep sw,
     if (j > b.jmax || k > b.kmax || i < 1 || i > b.imax) return;
     const int n = cid(b, i, j, k);
     double v[NRF];
+    SweepRaw up;
+    sweep_load<true, KE>(b, n, up);
     {   // predictor (PREDGS / PRKEGS): lower faces
         SweepRaw r;
         sweep_load<false, KE>(b, n, r);
@@ -2528,10 +2537,8 @@ __global__ void __launch_bounds__(PSW * TW) k_sweep_prep(Prm p, Blk b, Sweep sw,
         for (int f = 0; f < NRF; f++) __builtin_nontemporal_store((RT)v[f], &recp[st_row(st, tile, s, f) + lane]);
     }
     {   // corrector (DIAGGS + CORRGS / DIKEGS + COKEGS): upper faces
-        SweepRaw r;
-        sweep_load<true, KE>(b, n, r);
         SweepCell c;
-        corr_prep<KE>(p, r, c);
+        corr_prep<KE>(p, up, c);
         v[RC_FAC] = c.fac; v[RC_VOL] = c.vol; v[RC_MK] = c.dt1 * c.wk; v[RC_DT1] = c.dt1;
         v[RC_WI] = c.wi; v[RC_WJ] = c.wj; v[RC_SCINV] = c.scinv; v[RC_SCINP] = c.scinp;
         sc_put<KE>(c, v + RC_SC);
@@ -3095,7 +3102,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
     if (w == SW + CW) {
         // the halo wave: lane (word q, offset e along the face) takes word q of the edge
         // column e from the upstream tile's slots, J and K face alike.  The blocks of a step
-        // are copied to LDS HLEAD steps ahead (so that no step waits for its own loads); words
+        // are copied to LDS HLEAD + 1 steps ahead, in the first phase of the step before; words
         // that were still empty then (either 32-bit half, as a copy may race the store) are
         // polled.  The values of step s go to the exchange buffers' halo column in the second
         // phase of step s - 1.  At the end the wave empties the slots it has read for the
@@ -5002,7 +5009,7 @@ static int implicit_impl(ff_ctx *c, BlockRec *r, int level, bool divcp)
                              : (f32 ? k_sweep_wg<true, false, float> : k_sweep_wg<true, false>));
         const dim3 tpred(w1 ? TW : WGP * TW), tcorr(w1 ? TW : WGC * TW);
         // (forming the corrector's records on a side stream during the predictor's wavefront
-        // was measured slower: the latency-bound sweep loses more than the pass gains)
+        // gains nothing: 192x96x96 SST, the wavefront 350 -> 627 us and the pass 380 -> 420)
         rc = launch(c, "k_sweep_prep", prep, gp, dim3(PSW * TW), kp, b, r->sw, r->st, tp);
         if (rc) return rc;
         // the one-wave sweeps leave their halo slots filled: empty them for the next one

@@ -183,7 +183,7 @@ const char *ff_last_error(const ff_ctx *ctx);
  *   forms beforehand in the sweeps' step order (coalesced, the recurrence-independent work
  *   off the wavefront), six or seven waves per tile (three form one face's outgoing contribution
  *   each, the others stream the records into LDS and move what enters and leaves the tile);
- *   needs 2 x 56 + 8 doubles per cell and step of device memory per level (about 1 KB per
+ *   needs 2 x 48 + 8 doubles per cell and step of device memory per level (about 1 KB per
  *   cell), allocated on the block's first implicit stage.  FF_LUSGS_STAGED1: the same with
  *   one wave per tile. */
 #define FF_LUSGS_STAGED  3
