@@ -666,13 +666,16 @@ __global__ void __launch_bounds__(256) k_crosko(Prm p, Blk b, double *cdmax)
 // Also zeroes FUN1, SRK and the residuals DRO.. (ZEROZZ, RESIKE res3c.f:3668-3674, 3730) and
 // takes the maximum of SEPS, at least zero, over the linear index range FUN1KO scans
 // (turb3.f:7423-7428): an integer maximum, since the bits of non-negative doubles order as
-// their values (and a maximum is exact in any order).
-__global__ void __launch_bounds__(256) k_kw_round(Blk b, double *cdmax)
+// their values (and a maximum is exact in any order).  At most one workgroup of 16 waves per
+// CU, looping: the atomics all go to one address (96x72x50 10.6 us; with a workgroup per 256
+// cells 23, and 192x96x96 52 against 91).
+constexpr int KWR_THREADS = 1024, KWR_GRID = 256;
+__global__ void __launch_bounds__(KWR_THREADS) k_kw_round(Blk b, double *cdmax)
 {
-    __shared__ double sh[256];
-    int n = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double sh[KWR_THREADS / 64];
     double m = 0.0;
-    if (n < b.ntot) {
+    const int lo = cid(b, 1, 1, 1), hi = cid(b, b.imax, b.jmax, b.kmax);
+    for (int n = blockIdx.x * KWR_THREADS + threadIdx.x; n < b.ntot; n += gridDim.x * KWR_THREADS) {
         const double ro = FLD(b, FF_RO)[n];
         FLD(b, FF_RK)[n] = per_ro(FLD(b, FF_RK), FLD(b, FF_RO), n) * ro;
         FLD(b, FF_REPS)[n] = per_ro(FLD(b, FF_REPS), FLD(b, FF_RO), n) * ro;
@@ -680,15 +683,14 @@ __global__ void __launch_bounds__(256) k_kw_round(Blk b, double *cdmax)
         FLD(b, FF_SRK)[n] = 0.;
 #pragma unroll
         for (int q = 0; q < 7; q++) FLD(b, FF_DRO + q)[n] = 0.;
-        if (n >= cid(b, 1, 1, 1) && n <= cid(b, b.imax, b.jmax, b.kmax)) m = dmax(FLD(b, FF_SEPS)[n], m);
+        if (n >= lo && n <= hi) m = dmax(FLD(b, FF_SEPS)[n], m);
     }
-    sh[threadIdx.x] = m;
+    for (int h = 32; h > 0; h >>= 1) m = dmax(__shfl_xor(m, h), m);
+    if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = m;
     __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if (threadIdx.x < h) sh[threadIdx.x] = dmax(sh[threadIdx.x + h], sh[threadIdx.x]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && sh[0] > 0.) atomicMax((unsigned long long *)cdmax, (unsigned long long)__double_as_longlong(sh[0]));
+    if (threadIdx.x) return;
+    for (int w = 1; w < KWR_THREADS / 64; w++) m = dmax(sh[w], m);
+    if (m > 0.) atomicMax((unsigned long long *)cdmax, (unsigned long long)__double_as_longlong(m));
 }
 
 // FUN1KO (turb3.f:7430-7446) and PRODKE (turb3.f:4720-4787, with MAKE_EPS turb3.f:7913)
@@ -4832,7 +4834,9 @@ static int residual_impl(ff_ctx *c, BlockRec *r, int level, int m2, double *resi
         Prm kp = make_prm(&c->prm, level);
         // CROSKO, its rounding of RK/REPS, FUN1KO's floor, FUN1KO + PRODKE (res3c.f:3817-3994)
         if ((rc = launch(c, "k_crosko", k_crosko, cells_grid(b, 256), dim3(256), kp, b, r->kw_scr)) ||
-            (rc = launch(c, "k_kw_round", k_kw_round, all_grid(b), dim3(256), b, r->kw_scr)) ||
+            (rc = launch(c, "k_kw_round", k_kw_round,
+                         dim3(std::min((b.ntot + KWR_THREADS - 1) / KWR_THREADS, KWR_GRID)),
+                         dim3(KWR_THREADS), b, r->kw_scr)) ||
             (rc = launch(c, "k_fun1_prod", k_fun1_prod, cells_grid(b, 256), dim3(256), kp, b,
                          (const double *)r->kw_scr)))
             return rc;
