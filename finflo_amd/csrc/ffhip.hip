@@ -3076,10 +3076,13 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
     // Barriers of every wave: one at the start, two per step (after dn, after the contributions).
 
     if (w >= SW && w < SW + CW) {
-        // a copy wave.  The last read of record s is in the first phase of step s, the first
-        // one of record s + 1 in the second phase of step s: before the first barrier of step
-        // s record s + 1 must have arrived, of the copies issued by then (up to record
-        // s - 1 + RS) the last RS - 2 may still be in flight, and after it slot s is free.
+        // a copy wave.  The last read of record s is in the second phase of step s (wave 0's face),
+        // the first one of record s + 1 there too: slot s is free after the second barrier of
+        // step s, so its next copy starts in the first phase of step s + 1; before the first
+        // barrier of step s record s + 1 must have arrived, and of the copies issued by then
+        // (up to record s - 1 + RS) the last RS - 2 may still be in flight.  (A copy started a
+        // phase earlier overtakes wave 0's reads if that wave is held up, as by the
+        // instruction fetches of a first launch.)
         const int c = w - SW;
         auto copy = [&](int s) {
             ring_copy<RBYTES / CW>((const char *)(rec + st_row(st, tile, row(s), 0)) + c * (RBYTES / CW),
@@ -3092,9 +3095,9 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
         if (RS <= nsteps) vm_wait<NLD * (RS - 1)>(); else vm_wait<0>();
         wg_step_sync();
         for (int s = 0; s < nsteps; s++) {
+            if (s > 0 && s - 1 + RS < nsteps) copy(s - 1 + RS);
             if (s - 1 + RS < nsteps) vm_wait<NLD * (RS - 2)>(); else vm_wait<0>();
             wg_step_sync();
-            if (s + RS < nsteps) copy(s + RS);
             wg_step_sync();
         }
         vm_wait<0>();
