@@ -1394,7 +1394,7 @@ __global__ void __launch_bounds__(128) k_residual(Prm p, Blk b, WallDev wd)
 // extra phase.  I- and J-faces meet their two cells through LDS.  A face flux is the same
 // function of the same operands whichever cell forms it, so the differences are those of
 // k_residual bit for bit.
-constexpr int RI = 32, RJ = 8;     // the built-in (I, J) tile (launch_residual)
+constexpr int RI = 32, RJ = 8;     // the built-in (I, J) tile of most blocks (builtin_shape)
 
 template <int IFLUX, bool FNS, int RI, int RJ, int RKC>
 __global__ void __launch_bounds__(RI * RJ) k_residual_tile(Prm p, Blk b, WallDev wd, TileGrid tg)
@@ -4646,24 +4646,74 @@ int ff_turb(ff_ctx *c, int level, int block)
 // the same operands); they differ in occupancy, halo re-reads and how many workgroups a
 // small (coarse-level) block offers the 256 CUs.
 
-// The built-in shape: 32x8 (I, J) tiles of one K-plane, or of two where one plane per
-// workgroup would make more than RES_WGS1 workgroups.  A face flux takes a lone wave about
-// 4 us (divisions and loads in one long chain), and a workgroup of n planes runs 4n + 1 of
-// them one after another: short tiles keep that chain short and the chip full, at the price
-// of one more K-face per tile.  Measured (k-omega residual, us): 64x4x8 tiles / 32x8x1 /
-// 32x8x2 on 48x24x24 165 / 31 / 47, on 101x53x47 194 / 91 / 88, on 128x64x64 197 / 129 /
-// 133, on 160x80x80 354 / 277 / 266, on 192x96x96 551 / 475 / 459; laminar 118 / 23 / 33,
-// 143 / 70 / 67, 143 / 96 / 99, 258 / 191 / 185, 397 / 340 / 329.  The line lies between
-// 128x64x64 (2048 one-plane workgroups) and 160x80x80 (4000).
-constexpr int RES_WGS1 = 3072;
-template <typename K>
-static int launch_residual(ff_ctx *c, const char *name, K k1, K k2, const Prm &kp, const Blk &b,
-                           const WallDev &wd)
+// The built-in shape.  A face flux takes a lone wave about 4 us (divisions and loads in one
+// long chain), and a workgroup of n planes runs 4n + 1 of them one after another: 32x8 tiles
+// of one K-plane keep that chain short and the chip full, at the price of one more K-face per
+// tile; above RES_WGS1 such workgroups two planes.  Measured (k-omega residual, us): 64x4x8
+// tiles / 32x8x1 / 32x8x2 on 48x24x24 165 / 31 / 47, on 101x53x47 194 / 91 / 88, on
+// 128x64x64 197 / 129 / 133, on 160x80x80 354 / 277 / 266, on 192x96x96 551 / 475 / 459;
+// laminar 118 / 23 / 33, 143 / 70 / 67, 143 / 96 / 99, 258 / 191 / 185, 397 / 340 / 329;
+// 64x4x8 / built-in on 128x64x64, 160x80x80 and 192x96x96: van Leer 122 / 86, 215 / 160 and
+// 344 / 289, laminar FULLNS 214 / 174, 517 / 360 and 647 / 620, k-omega FULLNS 307 / 249,
+// 683 / 482 and 867 / 820.  The line lies between 128x64x64 (2048 one-plane workgroups) and
+// 160x80x80 (4000).
+//
+// On a large block with few J rows the rows of the last 8-row tile that have no cells are
+// lanes the chip lacks: from one row of tiles with more workgroups than 256 times the number of
+// such rows, blocks of one or two J rows take 64x2 tiles, and those that 64x4 tiles cover with
+// fewer lanes take these, laminar FULLNS 32x4.  k-omega / laminar / k-omega FULLNS / laminar
+// FULLNS, 64x4x8 tiles, 32x8 and these (us): 1024x1x256 225 144 333 258, 335 214 641 502, 131
+// 89 255 154; 1024x4x256 324 237 482 363, 432 302 791 618, 282 205 489 348; 1024x9x256 680 503
+// 1231 938, 825 596 1567 1200, 675 498 1228 804; 384x20x256 567 410 904 673, 557 398 1014 766,
+// 502 356 899 581.  Below that line idle rows cost nothing (101x25x47, 188 workgroups a row: 52
+// 40 97 with 32x8, 52 41 104 with 64x4; 192x44x96, 576 a row: 231 151 416, 234 154 423).
+// 64x4 tiles take four planes above RES_WGS4 workgroups (1024x12x192, 9216: 565 / 424 us
+// against 575 / 426 with two; 384x20x256, 7680: 517 / 376 against 497 / 354), FULLNS, with two
+// waves per SIMD for three, above RES_WGS1 (1024x4x256, 4096: 489 us against 498).
+constexpr long long RES_WGS1 = 3072, RES_WGS4 = 8192;      // one-plane workgroups of 256 threads
+
+static TileShape builtin_shape(const Blk &b, bool kw, bool ns)
 {
-    const int nx = (b.imax + RI - 1) / RI, ny = (b.jmax + RJ - 1) / RJ;
-    const bool two = (long long)nx * ny * b.kmax > RES_WGS1;
-    const TileGrid tg = tile_grid(nx, ny, two ? (b.kmax + 1) / 2 : b.kmax);
-    return launch(c, name, two ? k2 : k1, dim3(NXCD * tg.per), dim3(RI * RJ), kp, b, wd, tg);
+    auto wgs = [&](int ri, int rj) { return (long long)((b.imax + ri - 1) / ri) * ((b.jmax + rj - 1) / rj) * b.kmax; };
+    const long long rows = (b.jmax + RJ - 1) / RJ;
+    TileShape s{RI, RJ, 1};
+    if (wgs(RI, RJ) > 256 * rows * rows) {
+        if (b.jmax <= 2) s = {64, 2, 1};
+        else if (wgs(64, 4) < wgs(RI, RJ)) s = {ns && !kw ? 32 : 64, 4, 1};
+    }
+    const long long n = wgs(s.ri, s.rj) * (s.ri * s.rj) / 256;
+    if (n > RES_WGS1) s.rk = s.ri * s.rj == 256 && s.rj == 4 && (ns || n > RES_WGS4) ? 4 : 2;
+    return s;
+}
+
+// the kernels of the built-in shapes
+using ResKern = void (*)(Prm, Blk, WallDev, TileGrid);
+struct ResTile { TileShape s; ResKern k; };
+template <int IFLUX>
+constexpr ResTile kTileBuiltin[] = {
+    {{RI, RJ, 1}, k_residual_tile<IFLUX, false, RI, RJ, 1>}, {{RI, RJ, 2}, k_residual_tile<IFLUX, false, RI, RJ, 2>},
+    {{64, 4, 1}, k_residual_tile<IFLUX, false, 64, 4, 1>}, {{64, 4, 2}, k_residual_tile<IFLUX, false, 64, 4, 2>},
+    {{64, 4, 4}, k_residual_tile<IFLUX, false, 64, 4, 4>},
+    {{64, 2, 1}, k_residual_tile<IFLUX, false, 64, 2, 1>}, {{64, 2, 2}, k_residual_tile<IFLUX, false, 64, 2, 2>}};
+template <int IFLUX>
+constexpr ResTile kTileNsBuiltin[] = {
+    {{RI, RJ, 1}, k_residual_tile<IFLUX, true, RI, RJ, 1>}, {{RI, RJ, 2}, k_residual_tile<IFLUX, true, RI, RJ, 2>},
+    {{32, 4, 1}, k_residual_tile<IFLUX, true, 32, 4, 1>}, {{32, 4, 2}, k_residual_tile<IFLUX, true, 32, 4, 2>},
+    {{64, 2, 1}, k_residual_tile<IFLUX, true, 64, 2, 1>}, {{64, 2, 2}, k_residual_tile<IFLUX, true, 64, 2, 2>}};
+template <bool FNS>
+constexpr ResTile kKwBuiltin[] = {
+    {{RI, RJ, 1}, k_residual_kw<RI, RJ, 1, FNS>}, {{RI, RJ, 2}, k_residual_kw<RI, RJ, 2, FNS>},
+    {{64, 4, 1}, k_residual_kw<64, 4, 1, FNS>}, {{64, 4, 2}, k_residual_kw<64, 4, 2, FNS>},
+    {{64, 4, 4}, k_residual_kw<64, 4, 4, FNS>},
+    {{64, 2, 1}, k_residual_kw<64, 2, 1, FNS>}, {{64, 2, 2}, k_residual_kw<64, 2, 2, FNS>}};
+
+static int launch_residual(ff_ctx *c, const char *name, const ResTile *t, bool kw, bool ns, const Prm &kp,
+                           const Blk &b, const WallDev &wd)
+{
+    const TileShape s = builtin_shape(b, kw, ns);
+    while (t->s.ri != s.ri || t->s.rj != s.rj || t->s.rk != s.rk) t++;
+    const TileGrid tg = tile_grid((b.imax + s.ri - 1) / s.ri, (b.jmax + s.rj - 1) / s.rj, (b.kmax + s.rk - 1) / s.rk);
+    return launch(c, name, t->k, dim3(NXCD * tg.per), dim3(s.ri * s.rj), kp, b, wd, tg);
 }
 
 // the k-omega (kind 1) or laminar Roe (kind 0) residual kernel of shape s over block b
@@ -4848,10 +4898,8 @@ static int residual_impl(ff_ctx *c, BlockRec *r, int level, int m2, double *resi
         if (level == 1 && (rc = inlout_impl(c, r, level))) return rc;
         const int sh = fns ? -1 : tuned_shape(c, true, kp, b, wr.wd);
         rc = sh >= 0 ? launch_shape_any(c, sh, true, kp, b, wr.wd)
-             : fns   ? launch_residual(c, "k_residual_kw_ns", k_residual_kw<RI, RJ, 1, true>,
-                                       k_residual_kw<RI, RJ, 2, true>, kp, b, wr.wd)
-                     : launch_residual(c, "k_residual_kw", k_residual_kw<RI, RJ, 1>,
-                                       k_residual_kw<RI, RJ, 2>, kp, b, wr.wd);
+             : fns   ? launch_residual(c, "k_residual_kw_ns", kKwBuiltin<true>, true, true, kp, b, wr.wd)
+                     : launch_residual(c, "k_residual_kw", kKwBuiltin<false>, true, false, kp, b, wr.wd);
     } else {
         if (fns && (rc = gradients())) return rc;
         if ((rc = walls())) return rc;
@@ -4862,11 +4910,9 @@ static int residual_impl(ff_ctx *c, BlockRec *r, int level, int m2, double *resi
         if (sh >= 0) {
             rc = launch_shape_any(c, sh, false, kp, b, wr.wd);
         } else if (c->residual_mode == FF_RESIDUAL_TILES) {
-            auto k1 = fns ? (vl ? k_residual_tile<0, true, RI, RJ, 1> : k_residual_tile<1, true, RI, RJ, 1>)
-                          : (vl ? k_residual_tile<0, false, RI, RJ, 1> : k_residual_tile<1, false, RI, RJ, 1>);
-            auto k2 = fns ? (vl ? k_residual_tile<0, true, RI, RJ, 2> : k_residual_tile<1, true, RI, RJ, 2>)
-                          : (vl ? k_residual_tile<0, false, RI, RJ, 2> : k_residual_tile<1, false, RI, RJ, 2>);
-            rc = launch_residual(c, fns ? "k_residual_tile_ns" : "k_residual_tile", k1, k2, kp, b, wr.wd);
+            const ResTile *t = fns ? (vl ? kTileNsBuiltin<0> : kTileNsBuiltin<1>)
+                                   : (vl ? kTileBuiltin<0> : kTileBuiltin<1>);
+            rc = launch_residual(c, fns ? "k_residual_tile_ns" : "k_residual_tile", t, false, fns, kp, b, wr.wd);
         } else {
             auto kern = fns ? (vl ? k_residual<0, true> : k_residual<1, true>)
                             : (vl ? k_residual<0> : k_residual<1>);
