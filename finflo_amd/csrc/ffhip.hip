@@ -4728,9 +4728,12 @@ static int launch_shape(ff_ctx *c, bool kw, const Prm &kp, const Blk &b, const W
     return launch(c, "k_residual_tile", k_residual_tile<1, false, t.ri, t.rj, t.rk>, g, th, kp, b, wd, tg);
 }
 
+// a candidate shape, or the built-in one (s = -1)
 static int launch_shape_any(ff_ctx *c, int s, bool kw, const Prm &kp, const Blk &b, const WallDev &wd)
 {
     switch (s) {
+    case -1: return kw ? launch_residual(c, "k_residual_kw", kKwBuiltin<false>, true, false, kp, b, wd)
+                       : launch_residual(c, "k_residual_tile", kTileBuiltin<1>, false, false, kp, b, wd);
     case 0: return launch_shape<0>(c, kw, kp, b, wd);
     case 1: return launch_shape<1>(c, kw, kp, b, wd);
     case 2: return launch_shape<2>(c, kw, kp, b, wd);
@@ -4743,11 +4746,11 @@ static int launch_shape_any(ff_ctx *c, int s, bool kw, const Prm &kp, const Blk 
 }
 
 // The shape for this block and kind: from the table, or, on the first residual of such a
-// block outside a graph capture, by timing every candidate (one launch to warm up, three
-// timed with HIP events).  The k-omega kernel reads SEPS (the cross-diffusion CROSKO left
+// block outside a graph capture, by timing the built-in shape and every candidate (one launch
+// to warm up, three timed with HIP events).  The k-omega kernel reads SEPS (the cross-diffusion CROSKO left
 // there) before it overwrites it with the omega source, so SEPS is saved first and put back
 // before every launch; every other output is recomputed from unchanged inputs.  -1: the
-// built-in shapes.
+// built-in shape, by choice or untuned.
 static int tuned_shape(ff_ctx *c, bool kw, const Prm &kp, const Blk &b, const WallDev &wd)
 {
     if (c->force_shape >= 0) return c->force_shape;
@@ -4770,7 +4773,7 @@ static int tuned_shape(ff_ctx *c, bool kw, const Prm &kp, const Blk &b, const Wa
     bool ok = !kw || hipMemcpyAsync(save, seps, bytes, hipMemcpyDeviceToDevice, c->stream) == hipSuccess;
     int best = -1;
     double best_ms = 1e30;
-    for (int sh = 0; sh < NSHAPE && ok; sh++) {
+    for (int sh = -1; sh < NSHAPE && ok; sh++) {
         ok = restore() && launch_shape_any(c, sh, kw, kp, b, wd) == FF_OK;
         double tot = 0.;
         for (int rep = 0; rep < 3 && ok; rep++) {
@@ -4792,7 +4795,7 @@ static int tuned_shape(ff_ctx *c, bool kw, const Prm &kp, const Blk &b, const Wa
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (!ok) return -1;
-    if (best >= 0) c->tuned[key] = {best, best_ms};
+    c->tuned[key] = {best, best_ms};
     return best;
 }
 
@@ -4897,9 +4900,8 @@ static int residual_impl(ff_ctx *c, BlockRec *r, int level, int m2, double *resi
         if ((rc = walls())) return rc;
         if (level == 1 && (rc = inlout_impl(c, r, level))) return rc;
         const int sh = fns ? -1 : tuned_shape(c, true, kp, b, wr.wd);
-        rc = sh >= 0 ? launch_shape_any(c, sh, true, kp, b, wr.wd)
-             : fns   ? launch_residual(c, "k_residual_kw_ns", kKwBuiltin<true>, true, true, kp, b, wr.wd)
-                     : launch_residual(c, "k_residual_kw", kKwBuiltin<false>, true, false, kp, b, wr.wd);
+        rc = fns ? launch_residual(c, "k_residual_kw_ns", kKwBuiltin<true>, true, true, kp, b, wr.wd)
+                 : launch_shape_any(c, sh, true, kp, b, wr.wd);
     } else {
         if (fns && (rc = gradients())) return rc;
         if ((rc = walls())) return rc;
@@ -4960,7 +4962,8 @@ int ff_tuned_shape(const ff_ctx *c, int level, int block, int *shape, double *ms
     const Blk &b = it->second.dev;
     const auto t = c->tuned.find(std::make_tuple(b.imax, b.jmax, b.kmax, c->prm.iturb == 6 ? 1 : 0));
     if (t == c->tuned.end()) return FF_E_STATE;
-    const TileShape &sh = kTileShapes[t->second.first];
+    const int best = t->second.first;
+    const TileShape sh = best >= 0 ? kTileShapes[best] : builtin_shape(b, c->prm.iturb == 6, false);
     shape[0] = sh.ri; shape[1] = sh.rj; shape[2] = sh.rk;
     if (ms) *ms = t->second.second;
     return FF_OK;

@@ -213,9 +213,10 @@ const char *ff_last_error(const ff_ctx *ctx);
 #define FF_PREC_MIXED      1
 /*   FF_OPT_AUTOTUNE: 1 lets the library pick the tile shape of the residual kernels (the
  *   k-omega RESIKE kernel and the laminar Roe RESIDU kernel) per block size: on the first
- *   residual of a block of new dimensions outside a graph capture it times each of eight
- *   (I, J, K) tile shapes and keeps the fastest for every later residual of such a block.
- *   All shapes give the same results bit for bit.  0 (default): the built-in shapes. */
+ *   residual of a block of new dimensions outside a graph capture it times the built-in
+ *   (I, J, K) tile shape and each of eight others and keeps the fastest for every later
+ *   residual of such a block.  All shapes give the same results bit for bit.  0 (default):
+ *   the built-in shapes. */
 #define FF_OPT_AUTOTUNE    5
 /*   FF_OPT_TILE_SHAPE: 0-7 runs every residual in that candidate shape of the autotuner
  *   (for tests and measurements), -1 (default) leaves the choice to FF_OPT_AUTOTUNE. */
