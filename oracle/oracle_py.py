@@ -15,6 +15,7 @@ from finflo_amd.layout import bc_views, wall_views
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB = os.path.join(HERE, "libff_oracle.so")
 REFLIB = os.path.join(HERE, "_ref", "libfinflo_ref.so")
+REFDIR = "/root/reference"       # the reference's sources, where there are any
 
 _ora = None
 _ref = None
@@ -24,7 +25,7 @@ def build():
     """Compile the C restatement (and the reference library when the sources exist)."""
     import subprocess
     subprocess.check_call(["make", "-s", "-C", HERE, "all"])
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile(os.path.join(REFDIR, "charac.f")):
         subprocess.check_call(["make", "-s", "-C", HERE, "ref"])
 
 
