@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "ffhip_device.h"
+#include "ffring.h"
 
 using namespace ff;
 
@@ -3046,9 +3047,10 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
     constexpr int NV = KE ? 7 : 5, NS = KE ? 7 : 4;
     constexpr bool F32 = sizeof(RT) == 4;
     constexpr int NW = FWD ? WGC : WGP;
-    constexpr int RS = FWD ? (F32 ? 6 : 3) : (F32 ? 8 : 5);   // ring slots: RS - 1 steps of lead
+    constexpr int RS = ring_slots<FWD, F32>();
     constexpr int RBYTES = rbytes<RT>();
     constexpr int NLD = (RBYTES + (FWD ? DBYTES : 0)) / 1024 / CW;   // a copy wave's loads per step
+    static_assert(NLD == ring_loads<FWD, F32>(), "the ring's header counts the same loads");
     static_assert(NLD * (RS - 1) <= 63, "vmcnt range");
     static_assert(RBYTES / CW % 1024 == 0 && DBYTES / CW % 1024 == 0, "whole loads per copy wave");
     constexpr int XJ = TJ + 1;                          // row stride of the J exchange buffer
@@ -3076,13 +3078,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
     // Barriers of every wave: one at the start, two per step (after dn, after the contributions).
 
     if (w >= SW && w < SW + CW) {
-        // a copy wave.  The last read of record s is in the second phase of step s (wave 0's face),
-        // the first one of record s + 1 there too: slot s is free after the second barrier of
-        // step s, so its next copy starts in the first phase of step s + 1; before the first
-        // barrier of step s record s + 1 must have arrived, and of the copies issued by then
-        // (up to record s - 1 + RS) the last RS - 2 may still be in flight.  (A copy started a
-        // phase earlier overtakes wave 0's reads if that wave is held up, as by the
-        // instruction fetches of a first launch.)
+        // a copy wave
         const int c = w - SW;
         auto copy = [&](int s) {
             ring_copy<RBYTES / CW>((const char *)(rec + st_row(st, tile, row(s), 0)) + c * (RBYTES / CW),
@@ -3091,16 +3087,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
                 ring_copy<DBYTES / CW>((const char *)(st.dn + (((size_t)tile * nsteps + s) * NDN) * TW) + c * (DBYTES / CW),
                                        (char *)dring[s % RS] + c * (DBYTES / CW), lane);
         };
-        for (int s = 0; s < RS && s < nsteps; s++) copy(s);
-        if (RS <= nsteps) vm_wait<NLD * (RS - 1)>(); else vm_wait<0>();
-        wg_step_sync();
-        for (int s = 0; s < nsteps; s++) {
-            if (s > 0 && s - 1 + RS < nsteps) copy(s - 1 + RS);
-            if (s - 1 + RS < nsteps) vm_wait<NLD * (RS - 2)>(); else vm_wait<0>();
-            wg_step_sync();
-            wg_step_sync();
-        }
-        vm_wait<0>();
+        ring_copy_wave<RS, NLD>(nsteps, copy, [](auto n) { vm_wait<decltype(n)::value>(); }, wg_step_sync);
         return;
     }
 
@@ -3276,7 +3263,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
                 for (int m = 0; m < 3; m++) xs[m] = rc[((FWD ? RC_X : RP_X) + W * 3 + m) * TW];
                 if (FWD) aux = rc[(W == 0 ? RC_CP : RC_RHO) * TW];
             };
-            if (W > 0) {
+            if (ring_face_phase(W) == 1) {
                 __builtin_amdgcn_s_sleep(4);
                 read_face();
             }
@@ -3302,13 +3289,14 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
                 for (int m = 0; m < NB; m++) bv[m] = bs[m];
                 fb = basis_get(bv);
             };
-            if (W > 0) basis();
+            if (ring_face_phase(W) == 1) basis();
             wg_step_sync();
             // ---- second phase: the contribution across face W --------------------------
             if (W > 0) {
 #pragma unroll
                 for (int m = 0; m < NV; m++) dn[m] = xd[m][lane];
-            } else {
+            }
+            if (ring_face_phase(W) == 2) {
                 read_face();
                 __builtin_amdgcn_sched_barrier(0);
                 basis();

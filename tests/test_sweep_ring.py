@@ -1,35 +1,32 @@
-"""The record ring of the LU-SGS sweeps (k_sweep_wg): a copy into a slot starts after a barrier
-that follows the slot's last read, and a record has arrived before its first read.  The order of
-the kernel's phases is taken from its source, so that a change of one side alone is found."""
-import re
+"""The record ring of the LU-SGS sweeps (k_sweep_wg): a record has arrived in its slot before
+its first read, and the copy into a slot starts after a barrier that follows the slot's last read.
+A model on the CPU runs the copy waves' own loop and takes the readers' phases from the same
+header as the kernel; it finds a wait left out, a wait for one load too few and a copy a phase
+early."""
+import subprocess
 from pathlib import Path
 
 import pytest
 
-SRC = (Path(__file__).parents[1] / "finflo_amd/csrc/ffhip.hip").read_text()
+HERE = Path(__file__).parent
+STEPS = [15, 16, 22, 38, 214]        # IMAX + 14: one cell, two, a tile's worth, more
 
 
-def schedule():
-    """(phase in which a copy wave starts the copy of record s + RS, its step's distance from s),
-    and the phases in which wave 0 reads its face of record s, counted from step s."""
-    k = SRC[SRC.index("k_sweep_wg(Prm p"):SRC.index("constexpr int KI = 16, KJ = 4;")]
-    loop = re.search(r"wg_step_sync\(\);\s*for \(int s = 0; s < nsteps; s\+\+\) \{\s*(.*?)\n        \}", k, re.S).group(1)
-    m = re.search(r"copy\(s( - 1)? \+ RS\)", loop)
-    assert m, "the copy of the ring's next record"
-    phase = 1 + loop[:m.start()].count("wg_step_sync()")
-    copy = (1 if m.group(1) else 0, phase)
-    ahead = "read_face(ring[slot]" in k
-    return copy, (-1, 2) if ahead else (0, 2)
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("ring") / "model"
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", str(HERE / "sweep_ring_model.cpp"), "-o", str(exe)])
+    return lambda n, wait="0", early=0: subprocess.check_output([str(exe), str(n), str(wait), str(early)],
+                                                                text=True).splitlines()
 
 
-@pytest.mark.parametrize("n", [2, 8, 24, 200])
-@pytest.mark.parametrize("rs", [3, 5, 6, 8])
-def test_no_copy_before_the_last_read(rs, n):
-    copy, face = schedule()
-    for s in range(rs, n):
-        old = s - rs
-        start = (old + copy[0], copy[1])
-        # waves 1 and 2 read record s in the first phase of step s, wave 0 its increments'
-        # fields a step ahead and its face where the source says
-        last = max((old, 1), (old - 1, 2), (old + face[0], face[1]))
-        assert start > last, f"ring of {rs}: the copy of record {s} starts in {start}, last read in {last}"
+@pytest.mark.parametrize("n", STEPS)
+def test_schedule(model, n):
+    assert model(n) == ["ok"] * 4
+
+
+@pytest.mark.parametrize("n", STEPS)
+@pytest.mark.parametrize("mistake", [dict(wait="none"), dict(wait="1"), dict(early=1)],
+                         ids=["no_wait", "one_load_too_few", "copy_a_phase_early"])
+def test_mistakes_are_found(model, n, mistake):
+    assert all(line != "ok" for line in model(n, **mistake))
