@@ -3011,6 +3011,13 @@ __device__ __forceinline__ void wg_step_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The code that follows starts N instructions of 4 bytes behind a 64-byte boundary
+template <int N>
+__device__ __forceinline__ void code_place()
+{
+    asm volatile(".p2align 6\n.rept %0\ns_nop 0\n.endr" ::"n"(N));
+}
+
 // the tile ticket of a multi-wave workgroup: taken by its first lane, shared through LDS
 __device__ __forceinline__ int tile_ticket_wg(const Sweep &s, int *slot)
 {
@@ -3041,6 +3048,14 @@ __device__ __forceinline__ int tile_ticket_wg(const Sweep &s, int *slot)
 // themselves -> this form): 128x64x64 383 / 406 -> 194 / 216, 192x96x96 609 / 643 -> 337 / 378,
 // 48x24x24 130 / 138 -> 72 / 78; one tile of 192 cells takes 0.68 us a step, and crossing a
 // tile costs 8 steps and about 2 us.
+//
+// Where each wave's code lies relative to 32-byte windows decides up to a quarter of a sweep's
+// time (any wave's code moved by 0 to 15 instructions of 4 bytes: period 8), so that an edit
+// anywhere before it in the kernel moved the sweeps by as much.  So every wave's code starts at
+// the place that measured best (code_place); 128x64x64, best / worst place seen, us: predictor
+// laminar 170 / 223 (FP32 records 166 / 226), k-omega 183 / 231 (181 / 232), corrector 215 / 250
+// (183 / 230) and 226 / 245 (203 / 238).  A change to a wave's own code asks for its place to be
+// measured again.
 template <bool FWD, bool KE, typename RT = double>
 __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk b, Sweep sw, SweepSt st)
 {
@@ -3079,6 +3094,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
 
     if (w >= SW && w < SW + CW) {
         // a copy wave
+        code_place<FWD && F32 ? 6 : 3>();
         const int c = w - SW;
         auto copy = [&](int s) {
             ring_copy<RBYTES / CW>((const char *)(rec + st_row(st, tile, row(s), 0)) + c * (RBYTES / CW),
@@ -3099,6 +3115,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
         // polled.  The values of step s go to the exchange buffers' halo column in the second
         // phase of step s - 1.  At the end the wave empties the slots it has read for the
         // next sweep.
+        code_place<FWD ? 1 : 6>();
         constexpr int HLEAD = 0;
         const int e = lane % TK, q = lane / TK, qv = q < NV ? q : 0;
         const bool inj = q < NV && (FWD ? tj > 0 : tj + 1 < sw.ntj) && tk * TK + e + 1 <= b.kmax;
@@ -3173,6 +3190,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
         // complete: one column for every jj.  Lane (c, m) stores cell m of the run of column
         // jj = c in the first phase of the next step but one; the cell written meanwhile has a
         // slot of its own.  DRO/CP is formed here, off the compute waves.
+        code_place<6>();
         const int c = lane / 8, m8 = lane % 8;
         auto store = [&](int s) {
             const int ck = (s + 1 - c) & 7, q = s - c - ck - 7 + m8;
@@ -3195,6 +3213,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
 
     auto compute = [&](auto wave) __attribute__((always_inline)) {
         constexpr int W = decltype(wave)::value;
+        code_place<FWD ? (F32 ? (KE ? 6 : 7) : 4) : (W == 2 ? 0 : 4)>();
         // where this lane's contribution goes and where wave 0 finds its neighbours'
         const int wj = FWD ? kk * XJ + jj + 1 : kk * XJ + jj, rj = FWD ? wj - 1 : wj + 1;
         const int wk = FWD ? lane + TJ : lane, rk = FWD ? wk - TJ : wk + TJ;
