@@ -2650,8 +2650,8 @@ __device__ __forceinline__ bool half_empty(unsigned long long x)
 // words still missing at once, so a lane that has caught up with its upstream tile pays one
 // memory round trip per step, not one per word (the producer stores the words together).
 // Marker halves in words from the other two sources are ordinary values and are not
-// polled.  The staged sweeps leave their slots filled: a fill kernel empties all of them
-// after the sweep, which costs less than a device-coherent store per word on the
+// polled.  The one-wave staged sweeps leave their slots filled: a fill kernel empties all of
+// them after the sweep, which costs less than a device-coherent store per word on the
 // wavefront's critical path.
 template <int NV>
 __device__ __forceinline__ void halo_poll(unsigned long long *slot, unsigned int *err,
@@ -2978,21 +2978,25 @@ __global__ void __launch_bounds__(TW) k_corr_st(Prm p, Blk b, Sweep sw, SweepSt 
 }
 
 // ------------------------------------------------------------------------------------
-// The staged sweeps with six waves per tile.  Timestamps taken inside the one-wave kernels
-// above (s_memtime at the phase boundaries of every step, 192x96x96 level) split a step of
-// about 4,000 cycles into the face inputs (about 900: LDS reads of the exchange buffers and
+// The staged sweeps with six waves per tile, seven in the corrector.  Timestamps taken inside
+// the one-wave kernels above (s_memtime at the phase boundaries of every step, 192x96x96
+// level) split a step of about 4,000 cycles into the face inputs (about 900: LDS reads of the exchange buffers and
 // the halo ring, the marker tests), the recurrence and the three outgoing face
 // contributions (about 2,000) and the issue of the next record's LDS-DMA copies (about
 // 600: 28 loads of 1 KiB, which the memory pipeline accepts at about 64 bytes a clock).
 // All three are latencies on the step's critical path.  Here, per tile:
-// * waves 0-2 all form dn of the step from the same inputs, and wave f then forms only the
-//   contribution across face f (0: I, 1: J, 2: K) and leaves it in LDS; wave 1 publishes
-//   the J-face halo words and wave 2 the K-face ones;
+// * a step is two phases, each ended by a workgroup barrier.  In the first wave 0 forms the
+//   increments dn; in the second waves 0-2 form the contribution of dn across one face each
+//   (0: I, 1: J, 2: K), waves 1 and 2 leave theirs in LDS and publish the J-face and the
+//   K-face halo words;
 // * waves 3 and 4 issue the LDS-DMA copies (records, increments) and wait for them, wave 5
-//   takes the upstream tiles' halo words, so the three compute waves never wait on memory;
-// * one workgroup barrier per step separates a step's LDS writes from the next step's
-//   reads (the exchange buffers are double-buffered by step parity), and the other waves
-//   reach it only once what the next step reads is there.
+//   takes the upstream tiles' halo words and the corrector's wave 6 stores its results, so
+//   that the three compute waves never wait on memory;
+// * what passes between waves is written in one phase and read in another, so every buffer but
+//   the rings is single: xd (dn) is written in the first phase and read in the second; xj and
+//   xk (contributions, halo words) and obuf (results) are written in the second and read in the
+//   first of the next step; the halo staging is copied in the first and read in the second.  The
+//   record ring: ffring.h.
 // Arithmetic is that of k_pred_st / k_corr_st, operation for operation, so the results
 // are the same bit for bit.
 // ------------------------------------------------------------------------------------
@@ -3030,14 +3034,12 @@ __device__ __forceinline__ int tile_ticket_wg(const Sweep &s, int *slot)
 // (FWD = true: DRO/CP, D(rho k) and D(rho omega) times RO) on staged records.
 //
 // What bounds it: a step's latency times the I + J + K - 2 hyperplanes, plus the store-to-load
-// latency of every tile the wavefront crosses.  A step is two phases with a workgroup barrier
-// after each: in the first wave 0 forms the increments dn from its own I-contribution (kept in
-// registers) and the J- and K-contributions of the neighbour columns; in the second waves
-// 0-2 each form the contribution of dn across one face.  The three waves forming dn each for
-// itself needs one barrier less, but then each reads the 21 contributions and the increments'
-// fields from LDS at the same moment, 93 LDS instructions of 1 KiB a step against 62 here,
-// and the LDS becomes what the step waits for.  Everything else is kept off these
-// waves: they read the next record while they would wait (a wave's 15 outstanding LDS
+// latency of every tile the wavefront crosses.  Wave 0 alone forms the increments dn, from its
+// own I-contribution (kept in registers) and the J- and K-contributions of the neighbour
+// columns: the three waves forming dn each for itself needs one barrier less, but then each
+// reads the 21 contributions and the increments' fields from LDS at the same moment, 93 LDS
+// instructions of 1 KiB a step against 62 here, and the LDS becomes what the step waits for.
+// Everything else is kept off these waves: they read the next record while they would wait (a wave's 15 outstanding LDS
 // instructions are never exceeded), the exchange buffers have a ninth column or row that the
 // halo wave fills with the upstream tile's words (or that stays zero at the block's edge), so
 // that a lane reads its inputs at a constant offset with no test, and the corrector's results
@@ -3045,9 +3047,9 @@ __device__ __forceinline__ int tile_ticket_wg(const Sweep &s, int *slot)
 // on a cache line of its own: 64 partial lines per store held up the record copies).
 // Measured (k-omega, FP64 records, predictor / corrector, us; one phase of four waves per tile
 // that read the record after the barrier, tested every halo word and stored to the fields
-// themselves -> this form): 128x64x64 383 / 406 -> 194 / 216, 192x96x96 609 / 643 -> 337 / 378,
-// 48x24x24 130 / 138 -> 72 / 78; one tile of 192 cells takes 0.68 us a step, and crossing a
-// tile costs 8 steps and about 2 us.
+// themselves -> this form): 128x64x64 383 / 406 -> 184 / 226, 192x96x96 609 / 643 -> 342 / 409,
+// 48x24x24 130 / 138 -> 69 / 81; one tile of 192 cells takes 0.64 / 0.77 us a step, and crossing
+// a tile costs 8 steps and about 2 us.
 //
 // Where each wave's code lies relative to 32-byte windows decides up to a quarter of a sweep's
 // time (any wave's code moved by 0 to 15 instructions of 4 bytes: period 8), so that an edit
@@ -3069,7 +3071,7 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
     static_assert(NLD * (RS - 1) <= 63, "vmcnt range");
     static_assert(RBYTES / CW % 1024 == 0 && DBYTES / CW % 1024 == 0, "whole loads per copy wave");
     constexpr int XJ = TJ + 1;                          // row stride of the J exchange buffer
-    constexpr int HST = 4;                              // halo staging slots
+    constexpr int HST = 2;                              // halo staging slots
     constexpr int OS = 9, OST = TW + 4;                 // result slots per column, their stride
     __shared__ __attribute__((aligned(16))) RT ring[RS][NRF * TW];
     __shared__ __attribute__((aligned(16))) double dring[FWD ? RS : 1][NDN * TW];
@@ -3109,14 +3111,11 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
 
     if (w == SW + CW) {
         // the halo wave: lane (word q, offset e along the face) takes word q of the edge
-        // column e from the upstream tile's slots, J and K face alike.  The blocks of a step
-        // are copied to LDS HLEAD + 1 steps ahead, in the first phase of the step before; words
-        // that were still empty then (either 32-bit half, as a copy may race the store) are
-        // polled.  The values of step s go to the exchange buffers' halo column in the second
-        // phase of step s - 1.  At the end the wave empties the slots it has read for the
-        // next sweep.
+        // column e from the upstream tile's slots, J and K face alike.  The blocks of step s
+        // are copied to LDS in the first phase of step s - 1; words that were still empty then
+        // (either 32-bit half, as a copy may race the store) are polled.  The values go to the exchange buffers' halo column in that step's second
+        // phase.  At the end the wave empties the slots it has read for the next sweep.
         code_place<FWD ? 1 : 6>();
-        constexpr int HLEAD = 0;
         const int e = lane % TK, q = lane / TK, qv = q < NV ? q : 0;
         const bool inj = q < NV && (FWD ? tj > 0 : tj + 1 < sw.ntj) && tk * TK + e + 1 <= b.kmax;
         const bool ink = q < NV && (FWD ? tk > 0 : tk + 1 < sw.ntk) && tj * TJ + e + 1 <= b.jmax;
@@ -3129,13 +3128,11 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
             halo_dma(sj + d, hst[s % HST][0], lane);
             halo_dma(sk + d, hst[s % HST][1], lane);
         };
-        static_assert(HST > HLEAD + 1, "a staging slot is read before it is filled again");
         const int xjo = e * XJ + (FWD ? 0 : TJ), xko = (FWD ? 0 : TJ * TK) + e;
-        // step s: the copies of the HLEAD later steps have been issued after its own
         auto take = [&](int s) {
             const int i = diag(s) - e + 1;
             const bool live = i >= 1 && i <= b.imax, lj = inj && live, lk = ink && live;
-            vm_wait<2 * HLEAD>();
+            vm_wait<0>();
             unsigned long long vj = __double_as_longlong(hst[s % HST][0][qv * TK + e]);
             unsigned long long vk = __double_as_longlong(hst[s % HST][1][qv * TK + e]);
             bool pj = lj && half_empty(vj), pk = lk && half_empty(vk);
@@ -3160,11 +3157,11 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
             if (lj) xj[qv][xjo] = __longlong_as_double((long long)vj);
             if (lk) xk[qv][xko] = __longlong_as_double((long long)vk);
         };
-        for (int m = 0; m <= HLEAD; m++) copy(m);
+        copy(0);
         take(0);
         wg_step_sync();
         for (int s = 0; s < nsteps; s++) {
-            copy(s + 1 + HLEAD);
+            copy(s + 1);
             wg_step_sync();
             if (s + 1 < nsteps) take(s + 1);
             wg_step_sync();
@@ -3188,8 +3185,8 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
         // the store wave.  Column (jj, kk) leaves its cell q = s - jj - kk of step s in slot
         // q % OS.  After the steps with s - jj - kk = 7 (mod 8) a run of eight cells is
         // complete: one column for every jj.  Lane (c, m) stores cell m of the run of column
-        // jj = c in the first phase of the next step but one; the cell written meanwhile has a
-        // slot of its own.  DRO/CP is formed here, off the compute waves.
+        // jj = c in the first phase of the next step, while no results are written.  DRO/CP is
+        // formed here, off the compute waves.
         code_place<6>();
         const int c = lane / 8, m8 = lane % 8;
         auto store = [&](int s) {
@@ -3272,7 +3269,9 @@ __global__ void __launch_bounds__((FWD ? WGC : WGP) * TW) k_sweep_wg(Prm p, Blk 
                 __builtin_amdgcn_sched_barrier(0);
             }
             // the face's fields: waves 1 and 2 read them behind wave 0's inputs, which the
-            // step waits for, wave 0 its own in the second phase
+            // step waits for, wave 0 its own in the second phase.  The delay of 256 clocks
+            // lets wave 0's reads go first: 128x64x64 k-omega predictor 190 us without, 184 with,
+            // 195 with twice as much (FP32 records 189, 183, 190; corrector 213, 206, 215)
             auto read_face = [&]() __attribute__((always_inline)) {
 #pragma unroll
                 for (int m = 0; m < NS; m++) sv[m] = rc[((FWD ? RC_SC : RP_SC) + m) * TW];
