@@ -4041,16 +4041,17 @@ struct ff_ctx {
 static void mlp_free(MlpRec &r);
 static int earsm_mlp_pass(ff_ctx *c, const Blk &b);
 
-// The fixed device scratch of ff_residual_noalloc: the RESL2 partials and sums and the
-// per-workgroup SEPS maxima of the k-omega residual, 36,680 doubles (about 287 KB) that
-// every GPU the library runs on holds until the process ends.  In host code `scratch`
+// The fixed device scratch of ff_residual_noalloc: the RESL2 partials and sums and the SEPS
+// maximum of the k-omega residual, 3,600 doubles (about 29 KB) that every GPU the library
+// runs on holds until the process ends.  In host code `scratch`
 // names a host-side stand-in; the device address comes from hipGetSymbolAddress, taken
 // once per device when a context is created there, and only that address is passed on.
 constexpr int NA_RED_PARTS = 512;                       // RESL2: 7 partials each
-constexpr int NA_KW_PARTS = 32768;                      // SEPS maxima: 256 entries each
 constexpr size_t NA_OFF_OUT = 7 * NA_RED_PARTS;         // RESL2 sums (8)
-constexpr size_t NA_OFF_KW = NA_OFF_OUT + 8;            // SEPS maxima (NA_KW_PARTS + 1)
-constexpr size_t NA_SCRATCH = NA_OFF_KW + NA_KW_PARTS + 8;
+constexpr size_t NA_OFF_KW = NA_OFF_OUT + 8;            // SEPS maximum
+constexpr size_t NA_SCRATCH = NA_OFF_KW + 8;
+// the k-omega blocks it takes: a limit of the call that callers know, not of the array
+constexpr int NA_KW_ENTRIES = 8388608;
 static __device__ __align__(256) double scratch[NA_SCRATCH];
 constexpr int NA_MAX_DEVICES = 64;
 static double *g_scratch_dev[NA_MAX_DEVICES];
@@ -4994,7 +4995,7 @@ int ff_residual_noalloc(ff_ctx *c, int level, const ff_block *dev, int m2, doubl
     r.level = level;
     r.dev = make_blk(dev);
     if (c->prm.iturb == 6) {
-        if ((r.dev.ntot + 255) / 256 > NA_KW_PARTS)
+        if (r.dev.ntot > NA_KW_ENTRIES)
             return fail(c, FF_E_ARG, "ff_residual_noalloc: the k-omega residual takes blocks of at most "
                         "8388608 entries including ghost layers (this one has %s)",
                         std::to_string(r.dev.ntot).c_str());

@@ -450,8 +450,8 @@ int  ff_dromax(ff_ctx *ctx, int block, int idrxx, double *dromax, int *ixerr, in
 
 /* ff_residual of a block given directly as caller-owned device arrays (the field pointers
  * of `dev` are device addresses), with no registration and no device allocation: every
- * scratch buffer (the RESL2 partials and sums, the k-omega SEPS maxima) lives in a fixed
- * device array of the library, 36,680 doubles (about 287 KB) that each GPU the library
+ * scratch buffer (the RESL2 partials and sums, the k-omega SEPS maximum) lives in a fixed
+ * device array of the library, 3,600 doubles (about 29 KB) that each GPU the library
  * runs on holds until the process ends.  No counterpart in the reference (RESIDI
  * ns3c.f:2355 is the computation); it is for callers that cannot allocate device memory:
  * code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.

@@ -1,7 +1,7 @@
 """ff_residual_noalloc (every scratch buffer in the library's fixed device array, no
 registration, no allocation) against ff_residual on a registered block, through the C-ABI:
 two calls in a row on the same context, the second on a smaller block, bit for bit in
-every field and in the RESL2 sums; and the size limit of the fixed array."""
+every field and in the RESL2 sums; and the call's limit on a k-omega block's size."""
 import ctypes as C
 
 import numpy as np
@@ -49,7 +49,7 @@ def test_residual_noalloc_matches_registered(hip_device, iturb):
         assert not bad, f"fields differ: {bad}"
         np.testing.assert_array_equal(r2, r1)
         assert np.all(r1[:5] > 0)
-    # beyond the fixed array: a k-omega block of more than 8,388,608 entries is refused
+    # beyond the limit: a k-omega block of more than 8,388,608 entries is refused
     # before anything runs (the pointers are never read)
     if iturb:
         big = blk.view_struct(base=t2.data_ptr())
