@@ -4767,6 +4767,11 @@ static int tuned_shape(ff_ctx *c, bool kw, const Prm &kp, const Blk &b, const Wa
     if (it != c->tuned.end()) return it->second.first;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return -1;
+    // on a stream of the pool the blocks before this one are still at work: timed beside them
+    // the candidates would be compared under different loads
+    if (c->in_pool)
+        for (hipStream_t q : c->pool)
+            if (q && hipStreamSynchronize(q) != hipSuccess) return -1;
     const size_t bytes = sizeof(double) * (size_t)b.ntot;
     double *seps = kw ? FLD(b, FF_SEPS) : nullptr, *save = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
