@@ -110,7 +110,7 @@ KERNELS = ("k_residual_kw", "k_residual_tile", "k_residual", "k_pred_tiles", "k_
            "k_turb_sst", "k_derfun", "k_crosko", "k_kw_round",
            "k_fun1_prod", "k_fin", "k_zero", "k_fill_slots",
            "k_save_old", "k_divcp", "k_resl2_part", "k_resl2_final", "k_restrict",
-           "k_forcing", "k_prolong", "k_ddadi", "k_ddadi_end", "k_reflec")
+           "k_forcing", "k_prolong", "k_ddadi", "k_reflec")
 
 
 def make_workload(name="sst-mg", seed=0):

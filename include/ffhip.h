@@ -222,7 +222,7 @@ const char *ff_last_error(const ff_ctx *ctx);
  *   (for tests and measurements), -1 (default) leaves the choice to FF_OPT_AUTOTUNE. */
 #define FF_OPT_TILE_SHAPE  6
 /*   FF_OPT_BLOCK_STREAMS: 1 makes ff_vcycle_blocks run the blocks' V-cycles of a cycle side
- *   by side, block n on the n mod 8-th stream of a pool forked from the context's stream and
+ *   by side, block n on the n mod 32-th stream of a pool forked from the context's stream and
  *   joined back before the level-1 exchange, so that the small blocks' launches and sweep
  *   wavefronts overlap instead of leaving most of the chip idle.  The blocks of a cycle are
  *   independent (each reads only its own ghost cells, which the exchange refreshes after
